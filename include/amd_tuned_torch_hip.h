@@ -515,6 +515,16 @@ size_t atk_conv_wgrad_workspace_bytes(int64_t N, int64_t Ci, int64_t D, int64_t 
 int atk_conv_wgrad(const void* x, const void* dy, float* dw, int64_t N, int64_t Ci, int64_t D, int64_t H,
                    int64_t W, int64_t Co, int KD, int dtype, void* workspace, size_t ws_bytes, atk_stream_t stream);
 
+/* The same weight gradient, and the bias gradient db[co] = sum_{n,z,y,x} dy[n,co,z,y,x] when db
+ * is not null, from one pass over x and dy.  Any Ci and Co, any W >= 8, rows of any alignment,
+ * tensors under 2 GiB.  dw [Co, Ci, KD, 3, 3] and db [Co] are out_dtype: ATK_F32, or dtype
+ * (the fp32 sums rounded once).  ATK_UNSUPPORTED (and 0 workspace bytes) outside that. */
+size_t atk_conv_param_grads_workspace_bytes(int64_t N, int64_t Ci, int64_t D, int64_t H, int64_t W, int64_t Co,
+                                            int KD);
+int atk_conv_param_grads(const void* x, const void* dy, void* dw, void* db, int64_t N, int64_t Ci, int64_t D,
+                         int64_t H, int64_t W, int64_t Co, int KD, int dtype, int out_dtype, void* workspace,
+                         size_t ws_bytes, atk_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Layout conversion between channels-last and channels-first memory (replaces the strided
  * `.contiguous(memory_format=...)` copies around the channels-last conv candidates; the

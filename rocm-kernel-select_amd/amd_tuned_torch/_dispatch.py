@@ -405,10 +405,10 @@ def _dgrad_via_forward(grad_output, weight, pad_t, nd, fwd):
     return fwd(dy, wt, None, 1, pad_t, 1, 1)
 
 
-def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd):
-    """Weight gradient through the native kernel for stride-1, dilation-1, groups-1 'same'
-    convs with 3x3 (2D) or 3x3x3 / 1x3x3 (3D) kernels in 16-bit types; None otherwise (or when
-    the kernel declines the shape)."""
+def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd, bias_grad):
+    """(dw, db) through the native kernel for stride-1, dilation-1, groups-1 'same' convs with
+    3x3 (2D) or 3x3x3 / 1x3x3 (3D) kernels in 16-bit types, db (the sum of dy, in the weight's
+    dtype) only with `bias_grad`; None otherwise (or when the kernel declines the shape)."""
     if groups != 1 or isinstance(padding, str) or weight.dtype not in (torch.float16, torch.bfloat16):
         return None
     tup = _triple if nd == 3 else _pair
@@ -429,19 +429,21 @@ def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups,
         kd, x5, g5 = 1, input.unsqueeze(2), grad_output.unsqueeze(2)
     if g5.dtype != x5.dtype or tuple(g5.shape[2:]) != tuple(x5.shape[2:]):
         return None
+    out_dtype = weight.dtype if weight.dtype == x5.dtype else torch.float32
     try:
-        dw = _native.conv_wgrad(_to_ncdhw(x5), _to_ncdhw(g5), kd)
+        got = _native.conv_wgrad(_to_ncdhw(x5), _to_ncdhw(g5), kd, bias_grad=bias_grad, out_dtype=out_dtype)
     except _native.Unsupported:
         return None
-    return dw.reshape(weight.shape).to(weight.dtype)
+    dw, db = got if bias_grad else (got, None)
+    return dw.view(weight.shape).to(weight.dtype), None if db is None else db.to(weight.dtype)
 
 
 def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
     """(dx, dw, db) of a patched conv for `needs` = [dx, dw, db] wanted:
     * dx of a stride-1, dilation-1, groups-1 conv through `fwd` (the accelerated forward) on dy
       with transposed, flipped weights;
-    * dw of a 'same' 3x3(x3) conv in a 16-bit type through the native wgrad kernel;
-    * db as a reduction of dy once every other gradient is native;
+    * dw of a 'same' 3x3(x3) conv in a 16-bit type through the native wgrad kernel, db with it;
+    * db alone as a reduction of dy once every other gradient is native;
     * whatever is left through aten.convolution_backward, the op autograd uses unpatched."""
     stride, padding, dilation, groups, nd = conf
     needs = list(needs)
@@ -455,9 +457,11 @@ def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
             else:
                 gi = None
     if needs[1] and input.is_cuda:
-        gw = _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd)
-        if gw is not None:
+        got = _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd, needs[2])
+        if got is not None:
+            gw, gb = got
             needs[1] = False
+            needs[2] = needs[2] and gb is None
     if needs[2] and not needs[0] and not needs[1]:
         gb = grad_output.sum(dim=[0] + list(range(2, 2 + nd)), dtype=torch.float32).to(weight.dtype)
         needs[2] = False

@@ -45,6 +45,7 @@ EXPORTED_SYMBOLS = (
     "atk_group_norm_cl_fwd", "atk_group_norm_bwd_workspace_bytes",
     "atk_group_norm_bwd", "atk_conv_workspace_bytes",
     "atk_conv_fwd", "atk_conv_wgrad_workspace_bytes", "atk_conv_wgrad", "atk_transpose_last2",
+    "atk_conv_param_grads_workspace_bytes", "atk_conv_param_grads",
     "atk_dwconv1d_bwd", "atk_group_norm_noalloc_scratch_bytes", "atk_group_norm_fwd_noalloc",
     "atk_conv_packed_weight_bytes", "atk_conv_prepacked_workspace_bytes", "atk_conv_pack_weights",
     "atk_conv_fwd_prepacked", "atk_conv_fwd_prepacked_cl", "atk_conv_gn_stats_bytes", "atk_conv_gn_records",
@@ -198,6 +199,10 @@ def _declare(lib) -> None:
     lib.atk_conv_wgrad_workspace_bytes.restype = sz
     lib.atk_conv_wgrad.argtypes = [vp, vp, vp, i64, i64, i64, i64, i64, i64, i32, i32, vp, sz, vp]
     lib.atk_conv_wgrad.restype = i32
+    lib.atk_conv_param_grads_workspace_bytes.argtypes = [i64, i64, i64, i64, i64, i64, i32]
+    lib.atk_conv_param_grads_workspace_bytes.restype = sz
+    lib.atk_conv_param_grads.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i32, i32, i32, vp, sz, vp]
+    lib.atk_conv_param_grads.restype = i32
     lib.atk_transpose_last2.argtypes = [vp, vp, i64, i64, i64, i32, vp]
     lib.atk_transpose_last2.restype = i32
     lib.atk_dwconv1d_bwd.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i32, i32, i64, i32, vp, sz, vp]
@@ -1423,11 +1428,13 @@ def group_norm_apply(x: torch.Tensor, num_groups: int, weight: Optional[torch.Te
     return y
 
 
-def conv_wgrad(x: torch.Tensor, dy: torch.Tensor, kd: int) -> torch.Tensor:
-    """fp32 weight gradient [Co, Ci, kd, 3, 3] of a stride-1, dilation-1, 'same'-padded
+def conv_wgrad(x: torch.Tensor, dy: torch.Tensor, kd: int, *, bias_grad: bool = False,
+               out_dtype: torch.dtype = torch.float32):
+    """Weight gradient [Co, Ci, kd, 3, 3] of a stride-1, dilation-1, 'same'-padded
     (kd // 2, 1, 1) conv3d with kernel (kd, 3, 3), kd in {1, 3}: x [N, Ci, D, H, W] and
-    dy [N, Co, D, H, W] contiguous, one 16-bit dtype.  Raises Unsupported outside
-    Ci % 32 == 0, Co % 128 == 0, W % 16 == 0, W <= 64."""
+    dy [N, Co, D, H, W] contiguous, one 16-bit dtype; with `bias_grad` the pair (dw, db), db
+    [Co] the sum of dy, from the same pass.  The fp32 sums are rounded once to out_dtype (fp32
+    or x's).  Raises Unsupported for W < 8 or tensors of 2 GiB and more."""
     _require_cuda(x, dy)
     if x.dim() != 5 or dy.dim() != 5 or x.shape[0] != dy.shape[0] or x.shape[2:] != dy.shape[2:]:
         raise RuntimeError("conv_wgrad expects x [N, Ci, D, H, W] and dy [N, Co, D, H, W]")
@@ -1435,15 +1442,20 @@ def conv_wgrad(x: torch.Tensor, dy: torch.Tensor, kd: int) -> torch.Tensor:
         raise Unsupported("conv_wgrad: float16 / bfloat16 only")
     if not (x.is_contiguous() and dy.is_contiguous()):
         raise RuntimeError("conv_wgrad: x and dy must be contiguous")
+    if out_dtype not in (torch.float32, x.dtype):
+        raise RuntimeError("conv_wgrad: out_dtype must be float32 or x's dtype")
     N, Ci, D, H, W = x.shape
     Co = dy.shape[1]
-    if kd not in (1, 3) or Ci % 32 or Co % 128 or W % 16 or W > 64 or x.numel() == 0 or dy.numel() == 0:
-        raise Unsupported("conv_wgrad: needs kd in {1, 3}, Ci % 32, Co % 128, W % 16 == 0, W <= 64")
-    dw = torch.empty((Co, Ci, kd, 3, 3), dtype=torch.float32, device=x.device)
+    if kd not in (1, 3) or W < 8 or x.numel() == 0 or dy.numel() == 0:
+        raise Unsupported("conv_wgrad: needs kd in {1, 3} and W >= 8")
     L_ = lib()
-    nbytes = L_.atk_conv_wgrad_workspace_bytes(N, Ci, D, H, W, Co, kd)
+    nbytes = _cached_size(L_.atk_conv_param_grads_workspace_bytes, N, Ci, D, H, W, Co, kd)
+    if nbytes == 0:
+        raise Unsupported("conv_wgrad: shape outside the kernel's limits")
+    dw = torch.empty((Co, Ci, kd, 3, 3), dtype=out_dtype, device=x.device)
+    db = torch.empty((Co,), dtype=out_dtype, device=x.device) if bias_grad else None
     ws = workspace(x.device, "conv_wgrad", nbytes)
-    rc = L_.atk_conv_wgrad(_ptr(x), _ptr(dy), _ptr(dw), N, Ci, D, H, W, Co, kd, _DTYPE_CODE[x.dtype],
-                           _ptr(ws), ws.numel(), _stream(x))
+    rc = L_.atk_conv_param_grads(_ptr(x), _ptr(dy), _ptr(dw), _ptr(db), N, Ci, D, H, W, Co, kd,
+                                 _DTYPE_CODE[x.dtype], _DTYPE_CODE[out_dtype], _ptr(ws), ws.numel(), _stream(x))
     _check(rc, "conv_wgrad")
-    return dw
+    return (dw, db) if bias_grad else dw

@@ -441,6 +441,61 @@ def test_conv_wgrad_kernel_matches_float64(case, dtype):
     assert err <= 1e-4, f"max_rel_err {err:.3g}"
 
 
+PARAM_GRAD_CASES = [
+    # (N, Ci, Co, D, H, W, KD): one run per row, partial runs of 1 .. 7 positions, two column
+    # tiles, channel counts off 32, every number of waves per output-channel block, planes that
+    # one kz never meets
+    (1, 32, 32, 1, 1, 8, 1),
+    (2, 3, 64, 1, 9, 9, 1),
+    (1, 40, 96, 3, 7, 15, 3),
+    (1, 33, 130, 2, 5, 45, 3),
+    (2, 64, 64, 1, 33, 64, 1),
+    (1, 32, 160, 4, 11, 80, 3),
+    (1, 96, 256, 1, 6, 100, 3),
+    (3, 32, 33, 1, 17, 101, 1),
+    (1, 64, 32, 2, 130, 190, 1),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", PARAM_GRAD_CASES)
+def test_conv_param_grads_match_float64(case, dtype):
+    """atk_conv_param_grads (dw and db in one pass) against float64 on the CPU.  Products of
+    16-bit values are exact in fp32 and a chain adds at most a few thousand of them before the
+    partials are summed: within 1e-5 of the largest entry.  The 16-bit outputs are those sums
+    rounded once, and repeats are bit-identical."""
+    from amd_tuned_torch import _native
+    N, Ci, Co, D, H, W, KD = case
+    g = torch.Generator().manual_seed(Ci + Co + W)
+    x = torch.randn(N, Ci, D, H, W, generator=g).to(dtype)
+    dy = torch.randn(N, Co, D, H, W, generator=g).to(dtype)
+    dw, db = _native.conv_wgrad(x.cuda(), dy.cuda(), KD, bias_grad=True)
+    w = torch.zeros(Co, Ci, KD, 3, 3, dtype=torch.float64)
+    ref = torch.ops.aten.convolution_backward(dy.double(), x.double(), w, None, [1, 1, 1], [KD // 2, 1, 1],
+                                              [1, 1, 1], False, [0, 0, 0], 1, [False, True, False])[1]
+    assert O.max_rel_err(dw, ref) <= 1e-5
+    assert O.max_rel_err(db, dy.double().sum((0, 2, 3, 4))) <= 1e-5
+    dw16, db16 = _native.conv_wgrad(x.cuda(), dy.cuda(), KD, bias_grad=True, out_dtype=dtype)
+    assert torch.equal(dw16, dw.to(dtype)) and torch.equal(db16, db.to(dtype))
+    assert torch.equal(_native.conv_wgrad(x.cuda(), dy.cuda(), KD), dw)
+
+
+@pytest.mark.parametrize("W", [13, 16])
+def test_conv_param_grads_keep_infinities_local(W):
+    """An infinity in x reaches only the gradients whose sums contain it: the tap that would
+    need the position after a row's end does not see the row's last element."""
+    from amd_tuned_torch import _native
+    g = torch.Generator().manual_seed(W)
+    x = torch.randn(1, 32, 1, 5, W, generator=g).to(torch.bfloat16)
+    dy = torch.rand(1, 32, 1, 5, W, generator=g).add_(0.5).to(torch.bfloat16)
+    x[0, 7, 0, 2, W - 1] = float("inf")
+    dw = _native.conv_wgrad(x.cuda(), dy.cuda(), 1).cpu()
+    bad = ~torch.isfinite(dw)
+    assert bad[:, 7, 0, :, 1:].all() and not bad[:, 7, 0, :, 0].any()
+    bad[:, 7] = False
+    assert not bad.any()
+
+
 def test_conv_wgrad_full_size_c5a():
     """C5a's shape (1, 256 -> 256, 8x64x64, k3) bf16 against fp32 aten on the GPU."""
     from amd_tuned_torch import _native
