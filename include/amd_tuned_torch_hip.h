@@ -131,7 +131,7 @@ int atk_dwconv1d_bwd_weight(const void* x, const void* dy, float* dw, float* db,
  * src/causal-conv1d-amd/csrc/causal_conv1d.cpp:240-380 -> causal_conv1d_bwd.cu:100-235):
  * with z the recomputed fp32 pre-activation and g = dout * silu'(z) (dout without SiLU),
  *   dx[p] = sum_k w[k] g[p+K-1-k],  dw[c,k] = sum_{b,p} g[p] x[p-K+1+k],  db[c] = sum g.
- * x, dout, dx: [B, D, L] of `dtype`, contiguous, 16-byte aligned, L a multiple of 16 bytes;
+ * x, dout, dx: [B, D, L] of `dtype`, contiguous, any L, element-aligned;
  * w[c,k] at c*w_stride_c + k*w_stride_k in w_dtype (fp32 or `dtype`), bias [D] in w_dtype
  * or NULL; dw [D, K], db [D] fp32.  K in [2, 4].  The workspace (B*D*(K+1) floats) holds
  * per-row partials, summed over b in a fixed order.
@@ -235,8 +235,8 @@ int atk_dwconv1d_cl_bwd(const void* x, const void* dy, const void* w, void* dx, 
  * read once (atk_dwconv1d_fwd on dy plus atk_dwconv1d_bwd_weight read dy twice).  dw / db
  * may be NULL (dx only; db needs dw), and then no workspace is needed; otherwise the
  * workspace is atk_dwconv1d_bwd_weight_workspace_bytes(N, C, K), no initialisation.
- * K in [1, 5], pad_left <= 64; dx rows must be 16-byte aligned (L * sizeof(dtype) a
- * multiple of 16 and an aligned dx), else ATK_UNSUPPORTED.  Sums over n in a fixed order.
+ * K in [1, 5], pad_left <= 64; where dx rows are not 16-byte aligned (L * sizeof(dtype) no
+ * multiple of 16, or dx itself) pad_left < K, else ATK_UNSUPPORTED.  Sums over n in a fixed order.
  * ------------------------------------------------------------------------- */
 int atk_dwconv1d_bwd(const void* x, const void* dy, const void* w, void* dx, float* dw, float* db,
                      int64_t N, int64_t C, int64_t L, int K, int pad_left, int64_t L_out, int dtype,

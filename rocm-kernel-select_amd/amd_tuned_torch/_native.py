@@ -646,7 +646,7 @@ def causal_conv1d_bwd(x: torch.Tensor, dout: torch.Tensor, weight: torch.Tensor,
     """Fused backward of the causal (B, C, L) conv (pad K-1, output length L), width 2..4:
     (dx in x's dtype, dw (D, K) fp32, db (D,) fp32).  x, dout contiguous (B, D, L) of one dtype;
     weight (D, K) float32 or x's dtype, bias in the weight's dtype (recomputes the SiLU
-    pre-activation).  Raises Unsupported when L is not a multiple of 16 bytes."""
+    pre-activation).  Rows of any length and alignment."""
     _require_cuda(x, dout, weight, bias)
     if x.dim() != 3 or dout.shape != x.shape or dout.dtype != x.dtype or x.dtype not in _DTYPE_CODE:
         raise RuntimeError("causal_conv1d_bwd: x and dout must be (B, D, L) of one dtype")
@@ -722,7 +722,8 @@ def causal_conv1d_cl_bwd(x: torch.Tensor, dout: torch.Tensor, weight_dk: torch.T
 
 def _dwconv1d_backward_fused(dy: torch.Tensor, x: torch.Tensor, w: torch.Tensor, pad_left: int, needs):
     """(dx, dw, db) through atk_dwconv1d_bwd: x [N,C,L], dy [N,C,L_out], w [C,K] (x's dtype).
-    Raises Unsupported where the fused kernel declines (K > 5, unaligned dx rows, ...)."""
+    Raises Unsupported where the fused kernels decline (K > 5, unaligned dx rows with
+    pad_left >= K, ...)."""
     _require_cuda(x, dy, w)
     if x.dim() != 3 or dy.dim() != 3 or dy.shape[:2] != x.shape[:2] or w.shape[0] != x.shape[1]:
         raise RuntimeError("dwconv1d_backward expects x [N, C, L], dy [N, C, L_out], w [C, K]")

@@ -16,8 +16,8 @@ x.stride(2) > 1 is channel-last and runs the channels-last kernel, which also se
 layouts and by the decode step, as the reference dispatches the weight type separately
 (causal_conv1d.cpp:139-141,229,437); weights of another type are used in x's dtype.  The backward (the
 reference's causal_conv1d_bwd) is one fused channels-last kernel (dx, dweight, dbias, with the
-SiLU derivative from the recomputed fp32 pre-activation); the (B, C, L) layout composes the
-forward kernel on the flipped weights with the weight-gradient kernel.  The decode step
+SiLU derivative from the recomputed fp32 pre-activation), and one fused kernel for rows of any
+length in the (B, C, L) layout.  The decode step
 `causal_conv1d_update(x, conv_state, weight, bias, activation)` (interface :175-213) runs the
 library's update kernel.
 """
@@ -86,24 +86,7 @@ def _backward(x, weight, bias, dout, seq_idx, initial_states, dfinal, silu: bool
         # differentiate the function the forward computed: weights and bias as the kernel took them
         xc, g = x.contiguous(), dout.contiguous()
         wq, bq = _kernel_weight(weight, x, bias)
-        wq = wq.contiguous()
-        fused = None
-        try:
-            fused = _native.causal_conv1d_bwd(xc, g, wq, bq, silu=silu)
-        except _native.Unsupported:
-            fused = None
-        if fused is not None:
-            dx, dw, db = fused
-        elif silu:
-            # the SiLU derivative needs the fp32 pre-activation: run both kernels in fp32
-            xf, wf = xc.float(), wq.float()
-            z = _native.dwconv1d(xf, wf, bq.float() if bq is not None else None, K - 1, L)
-            gf = g.float() * _dsilu(z)
-            dx = _native.dwconv1d(gf, wf.flip(-1).contiguous(), None, 0, L).to(x.dtype)
-            dw, db = _native.dwconv1d_bwd_weight(xf, gf, K, K - 1)
-        else:
-            dx = _native.dwconv1d(g, wq.flip(-1).contiguous(), None, 0, L)
-            dw, db = _native.dwconv1d_bwd_weight(xc, g, K, K - 1)
+        dx, dw, db = _native.causal_conv1d_bwd(xc, g, wq, bq, silu=silu)
     dinit = None
     if initial_states is not None and want_dinit:
         # positions -(K-1)..-1: dinit[q] = sum_{t <= q} w[q - t] * g[t], g the gradient of the

@@ -1126,7 +1126,7 @@ int launch_update(const void* x, void* state, const void* w, const void* bias, v
 //   dx[p] = sum_j w[j] * g[p + H - j],  dw[j] = sum_u g[u] * x[u - H + j],  db = sum_u g[u].
 //
 // HBM-bound: x and dout are read once and dx written once (the halos are L1 / L2 hits).
-//  * A thread takes 2 * VEC consecutive positions per trip and loads its x and dout windows as
+//  * A thread takes CR_NV * VEC consecutive positions per trip and loads its x and dout windows as
 //    16-byte global loads at whatever address the row has (2-byte aligned loads are single
 //    instructions here), so no length needs a path of its own; only waves at the ends of a
 //    tensor, whose windows would leave it, load element by element, and only lanes at the ends
@@ -1136,9 +1136,17 @@ int launch_update(const void* x, void* state, const void* w, const void* bias, v
 //    quarters of each workgroup idle.
 //  * dw / db: per-thread sums, a fixed-order butterfly over the row's lanes (and LDS over its
 //    waves) into per-row partials, and the per-channel finalize above (sum over b in order).
-// [4, 2048, 2043] bf16, K = 4, SiLU, forward and backward: 294 -> 84 us (rows that are no
-// multiple of 16 bytes had taken fp32 copies and eight separate passes).
+// Causal backward, K = 4, SiLU, kernel and finalize: [4, 2048, 2043] bf16 29.6 us, 3.4 TB/s of x,
+// dout and dx (rows that are no multiple of 16 bytes took fp32 copies and eleven separate passes:
+// about 250 us); [4, 2048, 2048] 45.0 -> 29.8 us and config 2's [16, 2048, 8192] 367 -> 346 us
+// against a workgroup per row with 32 positions a thread.  Depthwise backward at rows of 2043:
+// 44.8 us in two passes -> 26.1 us.
 // ---------------------------------------------------------------------------------------
+// Vectors per thread and trip.  4 would recompute g for fewer positions past a thread's own
+// (35 / 32 of the work instead of 19 / 16) but measured 463 us against 385 on config 2's shape
+// with SiLU: fewer waves, and 64-byte strides between lanes.
+constexpr int CR_NV = 2;
+
 struct CrArgs {
   const void* x;
   const void* dy;
@@ -1150,6 +1158,7 @@ struct CrArgs {
   float* part;         // [rows][K+1], or null (dx only)
   int64_t rows;
   uint32_t D;
+  FastDiv div_d;
   int L, Lout, sh;
   int lpr_log2, trips;
 };
@@ -1173,19 +1182,39 @@ __device__ __forceinline__ void load_vecs(const T* base, int64_t e, int64_t tota
   }
 }
 
+// Lanes per row (log2) for `len` positions a row, T0 a thread: the fewest thread trips in all,
+// counting at least 2048 threads per CU; of equals the fewest lanes (a wave's prologue and its
+// butterfly are then shared by more trips), but whole waves where a row fills them.
+int pick_lanes(int64_t rows, int64_t len, int T0, int* trips) {
+  *trips = 1;
+  const int64_t per_row = (len + T0 - 1) / T0, fill = (int64_t)device_cu_count() * 2048;
+  int64_t best = 0;
+  int lanes = 3;
+  for (int lg = per_row >= 64 ? 6 : 3; lg <= 8; ++lg) {
+    const int64_t t = (per_row + (1 << lg) - 1) >> lg;
+    const int64_t cost = t * std::max(rows << lg, fill);
+    if (best == 0 || cost < best) {
+      best = cost;
+      lanes = lg;
+      *trips = (int)t;
+    }
+  }
+  return lanes;
+}
+
 template <typename T, int KT, bool SILU>
 __global__ __launch_bounds__(DW_NT) void conv1d_bwd_rows_kernel(CrArgs a) {
-  constexpr int VEC = 16 / sizeof(T);
+  constexpr int VEC = 16 / sizeof(T), NV = CR_NV;
   constexpr int H = KT - 1;
   static_assert(H <= VEC, "one halo vector on either side");
-  constexpr int T0 = 2 * VEC;                 // positions per thread and trip
-  constexpr int XV = SILU ? 4 : 3, GV = 3;    // x from p0 - VEC, g from p0
+  constexpr int T0 = NV * VEC;                         // positions per thread and trip
+  constexpr int XV = SILU ? NV + 2 : NV + 1, GV = NV + 1;  // x from p0 - VEC, g from p0
   __shared__ float red[(KT + 1) * (DW_NT / 64)];
   const int lpr = 1 << a.lpr_log2;
   const int lr = (int)threadIdx.x & (lpr - 1);
   const int64_t row = ((int64_t)blockIdx.x << (8 - a.lpr_log2)) + (threadIdx.x >> a.lpr_log2);
   const bool live = row < a.rows;
-  const uint32_t d = (uint32_t)((live ? row : 0) % a.D);
+  const uint32_t rr = live ? (uint32_t)row : 0u, d = rr - fdiv(rr, a.div_d) * a.D;
   float wv[KT], bv = 0.f;
 #pragma unroll
   for (int j = 0; j < KT; ++j) wv[j] = load_param(a.w, a.wdt, (int64_t)d * a.wc + (int64_t)j * a.wk);
@@ -1256,7 +1285,7 @@ __global__ __launch_bounds__(DW_NT) void conv1d_bwd_rows_kernel(CrArgs a) {
       accb += g[i];
     }
 #pragma unroll
-    for (int v = 0; v < 2; ++v) {
+    for (int v = 0; v < NV; ++v) {
       Vec16<T> r;
       r.raw = pack16<T>(o + v * VEC);
       const int p = p0 + v * VEC;
@@ -1303,48 +1332,34 @@ __global__ __launch_bounds__(DW_NT) void conv1d_bwd_rows_kernel(CrArgs a) {
 }
 
 template <typename T, int KT>
-void launch_cr_kt(const CrArgs& a, dim3 grid, int silu, hipStream_t s) {
+int launch_cr_kt(CrArgs a, int silu, hipStream_t s) {
+  a.lpr_log2 = pick_lanes(a.rows, std::max(a.L, a.Lout - a.sh), CR_NV * 16 / (int)sizeof(T), &a.trips);
+  const int64_t per_wg = 256 >> a.lpr_log2;
+  const dim3 grid((unsigned)((a.rows + per_wg - 1) / per_wg));
   if constexpr (KT >= 2 && KT <= 4) {
     if (silu) {
       hipLaunchKernelGGL((conv1d_bwd_rows_kernel<T, KT, true>), grid, dim3(DW_NT), 0, s, a);
-      return;
+      return check_launch("conv1d_bwd_rows_kernel");
     }
   }
   hipLaunchKernelGGL((conv1d_bwd_rows_kernel<T, KT, false>), grid, dim3(DW_NT), 0, s, a);
-}
-
-// Lanes per row: the fewest thread trips in all, counting at least 1024 threads per CU; of
-// equals the most lanes (longest runs of consecutive addresses).
-template <typename T>
-int launch_cr(CrArgs a, int K, int silu, hipStream_t s) {
-  constexpr int T0 = 2 * 16 / sizeof(T);
-  const int64_t per_row = ((int64_t)std::max(a.L, a.Lout - a.sh) + T0 - 1) / T0;
-  const int64_t fill = (int64_t)device_cu_count() * 1024;
-  int64_t best = 0;
-  for (int lg = 3; lg <= 8; ++lg) {
-    const int64_t trips = (per_row + (1 << lg) - 1) >> lg;
-    const int64_t cost = trips * std::max(a.rows << lg, fill);
-    if (best == 0 || cost <= best) {
-      best = cost;
-      a.lpr_log2 = lg;
-      a.trips = (int)trips;
-    }
-  }
-  const int64_t blocks = (a.rows + (256 >> a.lpr_log2) - 1) / (256 >> a.lpr_log2);
-  if (blocks > 0x7fffffff) return fail(ATK_UNSUPPORTED, "conv1d backward: grid too large");
-  const dim3 grid((unsigned)blocks);
-  switch (K) {
-    case 1: launch_cr_kt<T, 1>(a, grid, 0, s); break;
-    case 2: launch_cr_kt<T, 2>(a, grid, silu, s); break;
-    case 3: launch_cr_kt<T, 3>(a, grid, silu, s); break;
-    case 4: launch_cr_kt<T, 4>(a, grid, silu, s); break;
-    case 5: launch_cr_kt<T, 5>(a, grid, 0, s); break;
-    default: return fail(ATK_UNSUPPORTED, "conv1d backward: width %d outside [1, 5]", K);
-  }
   return check_launch("conv1d_bwd_rows_kernel");
 }
 
-int run_cr(const CrArgs& a, int K, int dtype, int silu, hipStream_t s) {
+template <typename T>
+int launch_cr(const CrArgs& a, int K, int silu, hipStream_t s) {
+  switch (K) {
+    case 1: return launch_cr_kt<T, 1>(a, 0, s);
+    case 2: return launch_cr_kt<T, 2>(a, silu, s);
+    case 3: return launch_cr_kt<T, 3>(a, silu, s);
+    case 4: return launch_cr_kt<T, 4>(a, silu, s);
+    case 5: return launch_cr_kt<T, 5>(a, 0, s);
+    default: return fail(ATK_UNSUPPORTED, "conv1d backward: width %d outside [1, 5]", K);
+  }
+}
+
+int run_cr(CrArgs a, int K, int dtype, int silu, hipStream_t s) {
+  a.div_d = make_fastdiv(a.D);
   switch (dtype) {
     case ATK_F32: return launch_cr<float>(a, K, silu, s);
     case ATK_F16: return launch_cr<_Float16>(a, K, silu, s);

@@ -250,6 +250,64 @@ def test_causal_bcl_autograd(dtype, silu, L, K):
     _grad_close(b.grad, db, "bcl dbias", 1e-5 if dtype == torch.float32 else 2e-3)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("L,K,B,D", [(1, 2, 1, 3), (7, 4, 2, 5), (15, 3, 3, 9), (17, 4, 2, 33), (65, 3, 4, 40),
+                                     (1021, 4, 2, 6), (1041, 2, 1, 7), (2043, 4, 1, 9), (8195, 4, 1, 2)])
+def test_causal_bcl_rows_of_any_length(dtype, L, K, B, D):
+    """Forward and fused backward on rows of every length class of the any-row kernels (part of
+    one thread's positions, several rows per wave, rows over several waves, several trips), from
+    base addresses off 16 bytes, against the float64 oracle; repeats are bit-identical."""
+    from amd_tuned_torch.causal_conv1d import causal_conv1d_fn
+    g = torch.Generator().manual_seed(L + K)
+
+    def off(t):  # the same values one element past an aligned base
+        buf = torch.zeros(t.numel() + 1, dtype=t.dtype, device="cuda")
+        buf[1:] = t.flatten().cuda()
+        return buf[1:].view(t.shape)
+
+    x = torch.randn(B, D, L, generator=g).to(dtype)
+    w, b = torch.randn(D, K, generator=g).cuda(), torch.randn(D, generator=g).cuda()
+    dy = torch.randn(B, D, L, generator=g).to(dtype)
+    got = []
+    for place in (lambda t: t.cuda(), off, off):
+        leaves = [place(x).requires_grad_(), w.clone().requires_grad_(), b.clone().requires_grad_()]
+        y = causal_conv1d_fn(*leaves, activation="silu")
+        got.append((y.detach(),) + torch.autograd.grad(y, leaves, place(dy)))
+    assert all(torch.equal(p, q) for p, q in zip(got[0], got[1]))
+    assert all(torch.equal(p, q) for p, q in zip(got[1], got[2]))
+    y, dx, dw, db = got[0]
+    ry, _ = O.causal_conv1d_states(x, w.cpu(), b.cpu(), silu=True)
+    rdx, rdw, rdb, _ = O.causal_conv1d_states_bwd(x, w.cpu(), b.cpu(), dy, silu=True)
+    _close(y, ry, dtype, "rows out")
+    _close(dx, rdx, dtype, "rows dx")
+    _grad_close(dw, rdw, "rows dweight", 1e-5 if dtype == torch.float32 else 2e-3)
+    _grad_close(db, rdb, "rows dbias", 1e-5 if dtype == torch.float32 else 2e-3)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("L,K,pad", [(5, 1, 0), (13, 2, 1), (29, 3, 1), (45, 4, 3), (77, 5, 2), (1033, 5, 4), (999, 4, 0)])
+def test_dwconv1d_backward_rows_of_any_length(dtype, L, K, pad):
+    """dx, dw and db of a padded depthwise conv in one pass where rows are not 16-byte aligned,
+    against the float64 oracle; an infinity in x reaches only the taps whose sums contain it."""
+    from amd_tuned_torch import _native
+    g = torch.Generator().manual_seed(L + K)
+    B, D = 3, 5
+    lo = L + 2 * pad - K + 1
+    x = torch.randn(B, D, L, generator=g).to(dtype)
+    w = torch.randn(D, K, generator=g).to(dtype)
+    dy = torch.randn(B, D, lo, generator=g).to(dtype)
+    dx, dw, db = _native._dwconv1d_backward_fused(dy.cuda(), x.cuda(), w.cuda(), pad, (True, True, True))
+    rdx, rdw, rdb = O.dwconv1d_bwd(x, w, dy, pad)
+    _close(dx, rdx, dtype, "rows dx")
+    _grad_close(dw, rdw, "rows dweight", 1e-5 if dtype == torch.float32 else 2e-3)
+    _grad_close(db, rdb, "rows dbias", 1e-5 if dtype == torch.float32 else 2e-3)
+    x[0, 1, L - 1] = float("inf")
+    _, dw, _ = _native._dwconv1d_backward_fused(dy.cuda(), x.cuda(), w.cuda(), pad, (True, True, True))
+    # tap j multiplies x[L - 1] by dy[L - 1 + pad - j], where that output exists
+    for j in range(K):
+        assert bool(torch.isfinite(dw[1, j])) == (not 0 <= L - 1 + pad - j < lo), j
+
+
 # channels checked against the float64 oracle in the full-size tests: first, last, a power of
 # two and two odd ones, over all 16 batch rows
 _SAMPLED_CHANNELS = [0, 1, 511, 1024, 2047]
