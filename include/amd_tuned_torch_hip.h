@@ -306,9 +306,8 @@ int atk_group_norm_fwd_noalloc(const void* x, const void* gamma, const void* bet
  * fused SiLU.  The reference serves this layout with Composable Kernel's groupnorm
  * (amd_tuned_torch/ck_norm_ops.py:9-27,93-103, picked by the contest in
  * amd_tuned_torch/_dispatch.py:2140-2200); same arithmetic and parameters as
- * atk_group_norm_fwd.  Needs (C/G)*sizeof(dtype) % 16 == 0, C*sizeof(dtype)/16 dividing
- * 256 (C <= 2048 for 16-bit types), G <= 256 and 16-byte aligned x / y (else
- * ATK_UNSUPPORTED).  Deterministic.
+ * atk_group_norm_fwd.  Needs C*sizeof(dtype) % 16 == 0, C*sizeof(dtype)/16 <= 256,
+ * G <= 256 and 16-byte aligned x / y (else ATK_UNSUPPORTED).  Deterministic.
  * Where 128 KB chunks cover every CU, one register-resident launch exchanges per-chunk
  * statistics between workgroups through the workspace (atk_group_norm_cl_workspace_bytes),
  * whose first bytes hold an epoch and counters that every launch leaves consistent: the
@@ -335,7 +334,7 @@ int atk_group_norm_cl_fwd(const void* x, const void* gamma, const void* beta, vo
  * x, dy, dx: [N, C, S] of `dtype`; gamma: [C] of `param_dtype` or NULL (ones);
  * dgamma / dbeta: [C] fp32.  Any of dx / dgamma / dbeta may be NULL.  The group
  * statistics are recomputed from x with the forward's eps.  Needs S * sizeof(dtype)
- * to be a multiple of 16 and 16-byte aligned x / dy / dx (else ATK_UNSUPPORTED).
+ * of at least 16 (else ATK_UNSUPPORTED); rows of any length and element alignment.
  * The first 16 KiB of the workspace (atk_group_norm_bwd_workspace_bytes) must be zero
  * before the first call that uses it; every call leaves them zero (per-group counters).
  * Sums over n are taken in a fixed order (deterministic).  Groups of up to 8192 16-byte

@@ -949,8 +949,8 @@ def group_norm_cl(input: torch.Tensor, num_groups: int, weight: Optional[torch.T
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """group_norm for channels-last input (NHWC / NDHWC memory, the layout the reference
     serves with CK, ck_norm_ops.py:9-27); the output keeps the input's memory format.
-    Raises Unsupported for shapes the kernel does not take (C/G not a multiple of 16 bytes,
-    C above 2048 16-bit channels, misaligned data)."""
+    Raises Unsupported for shapes the kernels do not take (C not a multiple of 16 bytes or
+    above 256 vectors, more than 256 groups, misaligned data)."""
     _require_cuda(input, weight, bias)
     if not is_channels_last(input):
         raise RuntimeError("group_norm_cl: input must be channels_last / channels_last_3d")
@@ -983,8 +983,8 @@ def group_norm_backward(dy: torch.Tensor, x: torch.Tensor, num_groups: int,
                         weight: Optional[torch.Tensor], eps: float, needs=(True, True, True)):
     """(dx, dgamma, dbeta) of group_norm(x, num_groups, weight, bias, eps) for dy: dx in x's
     dtype, dgamma / dbeta in fp32 ([C]); entries not asked for in `needs` are None.
-    x and dy contiguous NC[spatial]; raises Unsupported when the spatial size is not a
-    multiple of 16 bytes or a tensor is not 16-byte aligned."""
+    x and dy contiguous NC[spatial]; raises Unsupported when the spatial size is under 16
+    bytes."""
     _require_cuda(x, dy, weight)
     if x.dim() < 2 or dy.shape != x.shape:
         raise RuntimeError("group_norm_backward: dy must have x's shape (N, C, ...)")

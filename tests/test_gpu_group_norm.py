@@ -503,6 +503,84 @@ def test_group_norm_channels_last(dev, shape_g, dtype):
         _check(y.cpu().contiguous(), x, G, gm, bt, 1e-5, silu=silu, what=f"cl silu={silu}")
 
 
+# Rows that are no multiple of 16 bytes: shorter than two vectors, a group of exactly one vector,
+# every workgroup size of the resident kernel, groups past its 8192 vectors (two passes, a last
+# slice shorter than a vector among them)
+ANY_SHAPES = [
+    ((2, 6, 3, 3), 6),
+    ((1, 8, 1, 9), 4),
+    ((3, 40, 7, 7), 5),
+    ((2, 64, 45, 45), 8),
+    ((1, 32, 33, 61), 4),
+    ((1, 16, 3, 71, 53), 2),
+    ((2, 12, 211, 97), 3),
+    ((1, 4, 257, 255), 1),
+    ((1, 1, 1, 65537), 1),
+]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("case", ANY_SHAPES, ids=lambda s: "x".join(map(str, s[0])) + f"_g{s[1]}")
+def test_group_norm_rows_of_any_length(dev, case, dtype):
+    """Forward (with and without SiLU) and backward on rows of any length, from an aligned base
+    and one element off it (the same bits), against the float64 oracle."""
+    shape, G = case
+    nat = _native()
+    x, gm, bt = _inputs(shape, dtype, seed=sum(shape) + G)
+    dy = torch.randn(*shape, generator=torch.Generator().manual_seed(G)).to(dtype)
+
+    def off(t):
+        buf = torch.zeros(t.numel() + 1, dtype=t.dtype, device=dev)
+        buf[1:] = t.flatten().to(dev)
+        return buf[1:].view(t.shape)
+
+    vi = nat.variants(nat.OP_GROUP_NORM).index("twopass")
+    for silu in (False, True):
+        y = [nat.group_norm(p(x), G, gm.to(dev), bt.to(dev), 1e-5, silu=silu, variant=vi)
+             for p in (lambda t: t.to(dev), off, off)]
+        assert torch.equal(y[0], y[1]) and torch.equal(y[1], y[2])
+        _check(y[0].cpu(), x, G, gm, bt, 1e-5, silu=silu)
+    a = nat.group_norm_backward(dy.to(dev), x.to(dev), G, gm.to(dev), 1e-5, (True, True, True))
+    b = nat.group_norm_backward(off(dy), off(x), G, gm.to(dev), 1e-5, (True, True, True))
+    rdx, rdg, rdb = O.group_norm_bwd(x, G, gm, dy, 1e-5)
+    for dx, dg, db in (a, b):
+        assert O.max_rel_err(dx.cpu(), rdx) <= BAR[dtype]
+        assert O.max_rel_err(dg.cpu(), rdg) <= BWD_BAR_P[dtype]
+        assert O.max_rel_err(db.cpu(), rdb) <= BWD_BAR_P[dtype]
+
+
+# Channel counts and groups off the column map of the channels-last kernels: groups of part of a
+# vector, groups that straddle vectors, vector counts that do not divide the workgroup, one group,
+# as many groups as threads, one position, chunks with a partial last row block
+CL_ANY_SHAPES = [
+    ((2, 128, 16, 16), 32),
+    ((1, 192, 9, 11), 32),
+    ((3, 320, 7, 5), 32),
+    ((2, 24, 33, 3), 3),
+    ((1, 40, 64, 65), 5),
+    ((2, 48, 1, 1), 1),
+    ((1, 256, 3, 17, 19), 256),
+    ((1, 1000, 13, 4), 4),
+]
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("case", CL_ANY_SHAPES, ids=lambda s: "x".join(map(str, s[0])) + f"_g{s[1]}")
+def test_group_norm_channels_last_any_channels(dev, case, dtype):
+    shape, G = case
+    nat = _native()
+    x, gm, bt = _inputs(shape, dtype, seed=sum(shape) + G)
+    fmt = torch.channels_last if len(shape) == 4 else torch.channels_last_3d
+    xd = x.to(dev).contiguous(memory_format=fmt)
+    if not nat.is_channels_last(xd):
+        pytest.skip("one position: both layouts are the same")
+    for silu in (False, True):
+        y = nat.group_norm_cl(xd, G, gm.to(dev), bt.to(dev), 1e-5, silu=silu)
+        assert y.is_contiguous(memory_format=fmt)
+        assert torch.equal(y, nat.group_norm_cl(xd, G, gm.to(dev), bt.to(dev), 1e-5, silu=silu))
+        _check(y.cpu().contiguous(), x, G, gm, bt, 1e-5, silu=silu)
+
+
 # (shape, G, ATK_GN_CL_RESIDENT): which register-resident configuration the channels-last
 # forward takes ("0" = the three-kernel path).  With at least as many chunks per sample as
 # groups, one workgroup per group merges that group's chunk records (two-level); with fewer,
