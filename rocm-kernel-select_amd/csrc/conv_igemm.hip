@@ -218,11 +218,9 @@ struct PatchLoader {
   __device__ __forceinline__ static uint32_t dw(const uint4& v, int i) {
     return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
   }
-  __device__ __forceinline__ void store_quad(T* patch, int g, int total_quads, int tid, int nt) const {
+  __device__ __forceinline__ static void put_quad(T* dst, const uint4& c0, const uint4& c1, const uint4& c2,
+                                                  const uint4& c3) {
     constexpr int CBS = CB + VEC;
-    if (tid + g * nt >= total_quads) return;
-    T* dst = patch + qoff[g];
-    const uint4 &c0 = buf[4 * g], &c1 = buf[4 * g + 1], &c2 = buf[4 * g + 2], &c3 = buf[4 * g + 3];
     if constexpr (sizeof(T) == 2) {
       // position e of the 4 channels: halves e%2 of dword e/2 of each chunk
 #pragma unroll
@@ -237,6 +235,10 @@ struct PatchLoader {
       for (int e = 0; e < VEC; ++e)
         *reinterpret_cast<uint4*>(dst + e * CBS) = make_uint4(dw(c0, e), dw(c1, e), dw(c2, e), dw(c3, e));
     }
+  }
+  __device__ __forceinline__ void store_quad(T* patch, int g, int total_quads, int tid, int nt) const {
+    if (tid + g * nt >= total_quads) return;
+    put_quad(patch + qoff[g], buf[4 * g], buf[4 * g + 1], buf[4 * g + 2], buf[4 * g + 3]);
   }
 
   __device__ __forceinline__ void store(const IgArgs& a, T* patch, int total, int tid, int nt) const {
@@ -253,6 +255,77 @@ struct PatchLoader {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) dst[e * CBS] = v.e[e];
     }
+  }
+};
+
+// Patch staging of rows that are not 16-byte aligned (W no multiple of a chunk, or a misaligned
+// x), W >= VEC: the quad path above with each chunk loaded at the element address it has (2-byte
+// aligned 16-byte global loads are single instructions).  A row's last chunk, where it is
+// partial, is loaded as the row's last VEC elements and shifted down, zeros moving in, when it is
+// stored: no load leaves its row.  Chunks outside the patch or the input read zeros from g_zero16
+// (a global load has no bounds of its own).  Few waves hold partial chunks (a wave's quads share
+// their chunk column), so the shift is mostly skipped.  9 x 448 -> 96 channels, 3 x 31 x 55, k3 bf16:
+// 288 us with one load per element on the runtime tap schedule, 173 us here (150 us at width 56).
+__device__ uint4 g_zero16;
+
+template <typename T, int CB, int NTH, int XC>
+struct PatchLoaderRag : PatchLoader<T, CB, true, NTH, XC> {
+  using Base = PatchLoader<T, CB, true, NTH, XC>;
+  using Base::VEC;
+  using Base::NQ;
+  const char* xs;      // the sample
+  uint32_t part;       // bit g: quad g's chunks are partial
+  int shift;           // bits a partial chunk moves down by
+
+  __device__ __forceinline__ void init(const IgArgs& a, int iy0, int gx0, int total_quads, int tid, int nt) {
+    Base::init(a, iy0, gx0, total_quads, tid, nt);
+    part = 0;
+    const int s = VEC - a.W % VEC;  // elements missing in a partial chunk
+    shift = s * 8 * (int)sizeof(T);
+#pragma unroll
+    for (int g = 0; g < NQ; ++g) {
+      const int q = tid + g * nt;
+      const int cq = q % (CB / 4), rr = q / (CB / 4);
+      const int py = rr % a.PY, cx = rr / a.PY;
+      const int iy = iy0 + py, gx = gx0 + cx * VEC;
+      const bool p = q < total_quads && (unsigned)iy < (unsigned)a.H && gx >= 0 && gx < a.W && gx + VEC > a.W;
+      if (!p) continue;
+      part |= 1u << g;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        this->goff[g * 4 + k] -= (uint32_t)s;
+        this->clim[g * 4 + k] = cq * 4 + k;
+      }
+    }
+  }
+  __device__ __forceinline__ void load_fast(__amdgpu_buffer_rsrc_t, int u, uint32_t soff_el, int lim) {
+    const char* p = this->clim[u] < lim ? xs + (size_t)((this->goff[u] + soff_el) * (uint32_t)sizeof(T))
+                                        : reinterpret_cast<const char*>(&g_zero16);
+    typedef unsigned int u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
+    const u32x4_u v = *reinterpret_cast<const u32x4_u*>(p);
+    this->buf[u] = make_uint4(v.x, v.y, v.z, v.w);
+  }
+  __device__ __forceinline__ static uint4 moved(const uint4& v, int b) {
+    uint64_t lo = ((uint64_t)v.y << 32) | v.x, hi = ((uint64_t)v.w << 32) | v.z;
+    if (b >= 64) {
+      lo = hi;
+      hi = 0;
+      b -= 64;
+    }
+    lo = (lo >> b) | ((hi << 1) << (63 - b));
+    hi >>= b;
+    return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+  }
+  __device__ __forceinline__ void store_quad(T* patch, int g, int total_quads, int tid, int nt) const {
+    if (tid + g * nt >= total_quads) return;
+    uint4 c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = this->buf[4 * g + k];
+    if (part & (1u << g)) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[k] = moved(c[k], shift);
+    }
+    Base::put_quad(patch + this->qoff[g], c[0], c[1], c[2], c[3]);
   }
 };
 
@@ -310,13 +383,17 @@ struct PatchLoaderCL {
   }
 };
 
-template <typename T, int CB, bool VR, int NTH, int XC, bool CL>
+template <typename T, int CB, bool VR, int NTH, int XC, bool CL, bool RAG>
 struct LoaderSel {
   using type = PatchLoader<T, CB, VR, NTH, XC>;
 };
 template <typename T, int CB, bool VR, int NTH, int XC>
-struct LoaderSel<T, CB, VR, NTH, XC, true> {
+struct LoaderSel<T, CB, VR, NTH, XC, true, false> {
   using type = PatchLoaderCL<T, CB, NTH, XC>;
+};
+template <typename T, int CB, bool VR, int NTH, int XC>
+struct LoaderSel<T, CB, VR, NTH, XC, false, true> {
+  using type = PatchLoaderRag<T, CB, NTH, XC>;
 };
 
 // Bias of the workgroup's BN output channels as fp32 in LDS (zero without bias or when
@@ -1027,13 +1104,14 @@ __device__ __forceinline__ void store_tile_lds(const IgArgs& a, f32x16 (&acc)[FC
 // wave) then get KS waves per SIMD and a KS-times shorter chain of stage latencies, in one
 // launch and with no partial sums in memory.
 template <typename T, int WCO, int WSP, int FCO, int FSP, int CB, int XC, bool VR, int KHT, int KWT, bool EPI,
-          int KS = 1, bool CL = false, bool LEPI = false>
+          int KS = 1, bool CL = false, bool LEPI = false, bool RAG = false>
 __global__ __launch_bounds__(64 * WCO * WSP * KS)
 __attribute__((amdgpu_waves_per_eu(KS > 1 ? KS : ((FCO * FSP >= 8 && CB == 16) || XC > 1 ? 2 : 1))))
 void conv_igemm_kernel(IgArgs a) {
   static_assert(KS == 1 || KHT > 0, "the in-workgroup K split runs on the static tap schedule");
   static_assert(!CL || (KHT > 0 && VR && !EPI), "channels-last staging runs on the static tap schedule");
-  using Loader = typename LoaderSel<T, CB, VR, 64 * WCO * WSP, XC, CL>::type;
+  static_assert(!RAG || (KHT > 0 && VR && !EPI), "unaligned rows run on the static tap schedule");
+  using Loader = typename LoaderSel<T, CB, VR, 64 * WCO * WSP, XC, CL, RAG>::type;
   constexpr int NWG = WCO * WSP;          // waves per K group
   constexpr int NT = 64 * NWG;            // threads per K group (the tile's loaders)
   constexpr int KB = MfmaTraits<T>::KB, VEC = MfmaTraits<T>::VEC;
@@ -1114,6 +1192,8 @@ void conv_igemm_kernel(IgArgs a) {
   Loader ld;
   const int total_quads = total_chunks / 4;
   if constexpr (VR) ld.init(a, iy0, gx0, total_quads, tid, NT);
+  if constexpr (RAG)
+    ld.xs = reinterpret_cast<const char*>(static_cast<const T*>(a.x) + (int64_t)n * a.Ci * a.D * a.H * a.W);
   // stage s = (channel chunk cc, kernel plane kd), walked incrementally
   int cc = s_begin / a.KD, kd = s_begin - (s_begin / a.KD) * a.KD;
   const int iz_base = oz * a.sd - a.pd;
@@ -1523,6 +1603,9 @@ const IgVariant kIg[] = {
     // 64 output channels on large grids: 2x4 register tiles (half the weight loads per MFMA of
     // the 2x2 ones) over a 512-position tile, two workgroups per CU
     {"h_w14_f24_cb16x2", 0, 1, 4, 2, 4, 16, 2, 16},
+    // 128-position tiles with two K groups: shapes whose 256-position tiles leave CUs without one
+    {"h_w22_f22_cb32_k2", 0, 2, 2, 2, 2, 32, 1, 16, 2},
+    {"h_w22_f22_cb16_k2", 0, 2, 2, 2, 2, 16, 1, 16, 2},
 };
 constexpr int kNumIg = sizeof(kIg) / sizeof(kIg[0]);
 
@@ -1549,11 +1632,32 @@ int plan_ig(const ConvShape& p, int v, IgPlan& pl, bool unsplit = false) {
   a.KD = p.KD; a.KH = p.KH; a.KW = p.KW; a.sd = p.sd; a.sh = p.sh; a.sw = p.sw;
   a.pd = p.pd; a.ph = p.ph; a.pw = p.pw; a.dd = p.dd; a.dh = p.dh; a.dw = p.dw;
   a.Do = p.Do; a.Ho = p.Ho; a.Wo = p.Wo;
-  int tx = 1;
-  while (tx < p.Wo && tx < 64) tx <<= 1;
-  if (tx > pl.bm) tx = pl.bm;
-  a.TX = tx;
-  a.TY = pl.bm / tx;
+  // Tile rectangle: of the powers of two up to 64 columns that the loader's capacity and the LDS
+  // take, the one with the fewest tiles, the widest of equals.  One width for every plane left up
+  // to half of each tile outside it: an 80 x 45 plane under 64-column tiles takes 192 tiles of 256
+  // positions, 144 under 32-column ones (128 -> 128 channels, 8 planes, k3 bf16: with the
+  // 128-position tiles below 53.5 -> 47.8 us; 9 x 448 -> 96 channels on 31 x 56, 159 -> 150 us).
+  {
+    int64_t best = 0;
+    int tx = 1;
+    while (tx < p.Wo && tx < 64) tx <<= 1;
+    if (tx > pl.bm) tx = pl.bm;
+    const int maxc = (f32 ? vr.cb / 2 : vr.cb / 4) * vr.xc * 256 / ntg;  // PatchLoader::MAXC
+    a.TX = tx;
+    for (int t = tx; t >= std::min(tx, 8); t >>= 1) {
+      const int ty = pl.bm / t;
+      const int ncx = ((t - 1) * p.sw + (p.KW - 1) * p.dw + VEC) / VEC + 1;
+      const int py = (ty - 1) * p.sh + (p.KH - 1) * p.dh + 1;
+      const size_t lds = (size_t)2 * py * (ncx * VEC + 7) * (vr.cb + VEC) * es * vr.ks;
+      if (t != tx && (lds > (size_t)64 * 1024 * vr.ks || (int64_t)vr.cb * py * ncx > (int64_t)maxc * ntg)) continue;
+      const int64_t n = (int64_t)((p.Wo + t - 1) / t) * ((p.Ho + ty - 1) / ty);
+      if (best == 0 || n < best) {
+        best = n;
+        a.TX = t;
+      }
+    }
+  }
+  a.TY = pl.bm / a.TX;
   a.tiles_x = (p.Wo + a.TX - 1) / a.TX;
   a.tiles_y = (p.Ho + a.TY - 1) / a.TY;
   a.PX = (a.TX - 1) * p.sw + (p.KW - 1) * p.dw + 1;
@@ -1719,8 +1823,23 @@ int launch_ig_vr(const IgPlan& pl, hipStream_t s) {
   return launch_ig_kern<conv_igemm_kernel<T, WCO, WSP, FCO, FSP, CB, XC, VR, KHT, KWT, false, KS>>(pl, nt, s);
 }
 
+// Tiles with an instantiation for unaligned rows under a 3x3 plane: the ones that win at some size
+// there; the others keep the element-wise loader.
+constexpr bool rag_tile(int wco, int wsp, int fco, int fsp, int cb, int xc, int ks, int es) {
+  if (es == 4) return wco == 2 && ks == 1 && fco * fsp >= 2 && wsp == 2;
+  if (xc != 1) return false;
+  if (wco == 2 && wsp == 2) return fsp == 4 ? cb == 16 : fco == 2 ? cb == 32 : ks <= 2 && fsp == 1 && cb == 32;
+  return ks == 1 && ((wco == 2 && fsp == 4 && fco == 1) || (wco == 1 && wsp == 4));
+}
+
 template <typename T, int WCO, int WSP, int FCO, int FSP, int CB, int XC = 1, int KS = 1>
 int launch_ig_t(const IgPlan& pl, hipStream_t s) {
+  if constexpr (rag_tile(WCO, WSP, FCO, FSP, CB, XC, KS, sizeof(T))) {
+    if (pl.a.KH == 3 && pl.a.KW == 3 && !pl.cl && !pl.a.vec_rows && pl.a.W >= 16 / (int)sizeof(T) &&
+        !pl.a.resid && !pl.a.gn_parts && !pl.a.gn_onepass)
+      return launch_ig_kern<conv_igemm_kernel<T, WCO, WSP, FCO, FSP, CB, XC, true, 3, 3, false, KS, false, false, true>>(
+          pl, 64 * WCO * WSP * KS, s);
+  }
   if (pl.a.KH == 3 && pl.a.KW == 3 && pl.a.vec_rows)
     return launch_ig_vr<T, WCO, WSP, FCO, FSP, CB, XC, true, 3, 3, KS>(pl, s);
   if (pl.a.KH == 7 && pl.a.KW == 7 && pl.a.vec_rows)
@@ -1868,6 +1987,8 @@ int run_ig(const ConvShape& p, IgPlan& pl, const void* x, const void* wp, const 
       case 24: rc = launch_ig_t<T, 2, 2, 2, 4, 16, 1, 2>(pl, s); break;
       case 25: rc = launch_ig_t<T, 4, 1, 2, 2, 32, 1, 2>(pl, s); break;
       case 26: rc = launch_ig_t<T, 1, 4, 2, 4, 16, 2>(pl, s); break;
+      case 27: rc = launch_ig_t<T, 2, 2, 2, 2, 32, 1, 2>(pl, s); break;
+      case 28: rc = launch_ig_t<T, 2, 2, 2, 2, 16, 1, 2>(pl, s); break;
       default: return fail(ATK_EINVAL, "conv: bad variant");
     }
   } else {

@@ -441,6 +441,58 @@ def test_conv_wgrad_kernel_matches_float64(case, dtype):
     assert err <= 1e-4, f"max_rel_err {err:.3g}"
 
 
+# 3x3 planes over rows that are not 16-byte aligned: a row of one full and one partial chunk, partial
+# chunks of 1 .. 7 elements, in the first and in later column tiles, channel counts off the stage's
+# block, rows of exactly one chunk from a misaligned base
+RAGGED_CONV_CASES = [
+    (1, 16, 32, 1, 9, 9),
+    (2, 24, 64, 2, 11, 33),
+    (1, 33, 40, 1, 5, 62),
+    (1, 64, 128, 3, 7, 15),
+    (1, 8, 32, 1, 3, 131),
+    (2, 40, 96, 2, 6, 8),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", RAGGED_CONV_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_conv_unaligned_rows_every_tile(case, dtype):
+    """Every tile that takes the shape against the float64 oracle, from an aligned base and one
+    element off it; a NaN in one input row reaches only the outputs whose window holds it."""
+    from amd_tuned_torch import _native as nat
+    N, Ci, Co, D, H, W = case
+    g = torch.Generator().manual_seed(sum(case))
+    x = torch.randn(N, Ci, D, H, W, generator=g).to(dtype)
+    w = (torch.randn(Co, Ci, 3, 3, 3, generator=g) * (2.0 / (Ci * 27)) ** 0.5).to(dtype)
+    b = (torch.randn(Co, generator=g) * 0.1).to(dtype)
+    ref = O.conv3d(x, w, b, 1, 1, 1)
+    bar = 1e-5 if dtype == torch.float32 else 1e-2
+    xd = x.cuda()
+    off = torch.zeros(x.numel() + 1, dtype=dtype, device="cuda")
+    off[1:] = xd.flatten()
+    off = off[1:].view(x.shape)
+    bad = xd.clone()
+    bad[0, 0, 0, H // 2, W - 1] = float("nan")
+    ran = 0
+    for vi, name in enumerate(nat.variants(nat.OP_CONV)):
+        try:
+            y = nat.conv3d(xd, w.cuda(), b.cuda(), 1, 1, 1, variant=vi)
+        except nat.Unsupported:
+            continue
+        ran += 1
+        assert O.max_rel_err(y.cpu(), ref) <= bar, name
+        try:
+            y = nat.conv3d(off, w.cuda(), b.cuda(), 1, 1, 1, variant=vi)
+            assert O.max_rel_err(y.cpu(), ref) <= bar, name
+        except nat.Unsupported:  # a tile that takes aligned rows only
+            assert W % (16 // x.element_size()) == 0, name
+        z = torch.isnan(nat.conv3d(bad, w.cuda(), b.cuda(), 1, 1, 1, variant=vi))
+        want = torch.zeros_like(z)
+        want[0, :, :2, max(0, H // 2 - 1):H // 2 + 2, W - 2:] = True
+        assert torch.equal(z, want), name
+    assert ran >= 2
+
+
 PARAM_GRAD_CASES = [
     # (N, Ci, Co, D, H, W, KD): one run per row, partial runs of 1 .. 7 positions, two column
     # tiles, channel counts off 32, every number of waves per output-channel block, planes that
