@@ -524,6 +524,12 @@ int atk_conv_param_grads(const void* x, const void* dy, void* dw, void* db, int6
                          int64_t H, int64_t W, int64_t Co, int KD, int dtype, int out_dtype, void* workspace,
                          size_t ws_bytes, atk_stream_t stream);
 
+/* Weights of the forward conv that computes a stride-1 conv's input gradient: w [Co, Ci, taps]
+ * contiguous (taps = the kernel's positions in row-major order) -> wt [Ci, Co, taps] with the taps
+ * reversed, i.e. channels swapped and every spatial axis flipped.  2- or 4-byte dtype codes. */
+int atk_conv_dgrad_weight(const void* w, void* wt, int64_t Co, int64_t Ci, int64_t taps, int dtype,
+                          atk_stream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Layout conversion between channels-last and channels-first memory (replaces the strided
  * `.contiguous(memory_format=...)` copies around the channels-last conv candidates; the

@@ -399,7 +399,7 @@ def _dgrad_via_forward(grad_output, weight, pad_t, nd, fwd):
     """dL/dx of a stride-1, dilation-1 conv: the forward conv of dy with the weights swapped
     in (Co, Ci) and flipped in space, padding k-1-p -- so the input gradient runs on the
     forward path (and its per-shape contest) instead of a separate dgrad."""
-    wt = weight.transpose(0, 1).flip(list(range(2, 2 + nd))).contiguous()
+    wt = _native.conv_dgrad_weight(weight)
     # a channels-last dy goes in as is: the forward path converts it with the native transpose
     dy = grad_output if _channels_last(grad_output) else grad_output.contiguous()
     return fwd(dy, wt, None, 1, pad_t, 1, 1)

@@ -45,7 +45,7 @@ EXPORTED_SYMBOLS = (
     "atk_group_norm_cl_fwd", "atk_group_norm_bwd_workspace_bytes",
     "atk_group_norm_bwd", "atk_conv_workspace_bytes",
     "atk_conv_fwd", "atk_conv_wgrad_workspace_bytes", "atk_conv_wgrad", "atk_transpose_last2",
-    "atk_conv_param_grads_workspace_bytes", "atk_conv_param_grads",
+    "atk_conv_param_grads_workspace_bytes", "atk_conv_param_grads", "atk_conv_dgrad_weight",
     "atk_dwconv1d_bwd", "atk_group_norm_noalloc_scratch_bytes", "atk_group_norm_fwd_noalloc",
     "atk_conv_packed_weight_bytes", "atk_conv_prepacked_workspace_bytes", "atk_conv_pack_weights",
     "atk_conv_fwd_prepacked", "atk_conv_fwd_prepacked_cl", "atk_conv_gn_stats_bytes", "atk_conv_gn_records",
@@ -203,6 +203,8 @@ def _declare(lib) -> None:
     lib.atk_conv_param_grads_workspace_bytes.restype = sz
     lib.atk_conv_param_grads.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i32, i32, i32, vp, sz, vp]
     lib.atk_conv_param_grads.restype = i32
+    lib.atk_conv_dgrad_weight.argtypes = [vp, vp, i64, i64, i64, i32, vp]
+    lib.atk_conv_dgrad_weight.restype = i32
     lib.atk_transpose_last2.argtypes = [vp, vp, i64, i64, i64, i32, vp]
     lib.atk_transpose_last2.restype = i32
     lib.atk_dwconv1d_bwd.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i32, i32, i64, i32, vp, sz, vp]
@@ -1427,6 +1429,18 @@ def group_norm_apply(x: torch.Tensor, num_groups: int, weight: Optional[torch.Te
                                     int(variant), _stream(x))
     _check(rc, "group_norm_apply")
     return y
+
+
+def conv_dgrad_weight(weight: torch.Tensor) -> torch.Tensor:
+    """weight [Co, Ci, *k] -> [Ci, Co, *k] with every spatial axis flipped, contiguous: the weights
+    of the forward conv that computes the input gradient of a stride-1 conv."""
+    if not (weight.is_cuda and weight.is_contiguous() and weight.dtype in _DTYPE_CODE and weight.numel()):
+        return weight.transpose(0, 1).flip(list(range(2, weight.dim()))).contiguous()
+    Co, Ci = weight.shape[:2]
+    wt = torch.empty((Ci, Co) + tuple(weight.shape[2:]), dtype=weight.dtype, device=weight.device)
+    _check(lib().atk_conv_dgrad_weight(weight.data_ptr(), wt.data_ptr(), Co, Ci, weight.numel() // (Co * Ci),
+                                       _DTYPE_CODE[weight.dtype], _stream(weight)), "conv_dgrad_weight")
+    return wt
 
 
 def conv_wgrad(x: torch.Tensor, dy: torch.Tensor, kd: int, *, bias_grad: bool = False,

@@ -102,6 +102,20 @@ int launch_transpose(const TpArgs& a, bool vec_ok, hipStream_t s) {
   return check_launch("transpose_tile_kernel");
 }
 
+// wt[ci][co][taps - 1 - t] = w[co][ci][t]: the weights of the forward conv that computes the input
+// gradient, in one pass where torch took a flip and a copy.  A thread per element, writes
+// contiguous, reads in runs of `taps` (the tensors are small: 128 x 128 x 27 in bf16, 0.9 MB, is
+// bound by the launch).
+template <typename E>
+__global__ __launch_bounds__(256) void dgrad_weight_kernel(const E* __restrict__ w, E* __restrict__ wt, uint32_t Ci,
+                                                           uint32_t total, FastDiv div_co, FastDiv div_taps) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t q = fdiv(i, div_taps), t = i - q * div_taps.d;
+  const uint32_t ci = fdiv(q, div_co), co = q - ci * div_co.d;
+  wt[i] = w[(co * Ci + ci) * div_taps.d + div_taps.d - 1 - t];
+}
+
 }  // namespace
 }  // namespace atk
 
@@ -121,4 +135,26 @@ extern "C" int atk_transpose_last2(const void* in, void* out, int64_t B, int64_t
   a.in = in; a.out = out; a.B = B; a.R = R; a.C = C; a.tiles_c = tiles_c;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   return es == 4 ? launch_transpose<uint32_t>(a, vec_ok, s) : launch_transpose<uint16_t>(a, vec_ok, s);
+}
+
+extern "C" int atk_conv_dgrad_weight(const void* w, void* wt, int64_t Co, int64_t Ci, int64_t taps, int dtype,
+                                     atk_stream_t stream) {
+  using namespace atk;
+  if (!dtype_ok(dtype)) return fail(ATK_EINVAL, "conv dgrad weight: unknown dtype code %d", dtype);
+  if (Co <= 0 || Ci <= 0 || taps <= 0) return fail(ATK_EINVAL, "conv dgrad weight: bad sizes");
+  if (!w || !wt || w == wt) return fail(ATK_EINVAL, "conv dgrad weight: null or aliasing pointer");
+  constexpr int64_t lim = (int64_t)1 << 30;
+  if (Co >= lim || Ci >= lim || taps >= lim || Co * Ci >= lim || Co * Ci * taps >= lim)
+    return fail(ATK_UNSUPPORTED, "conv dgrad weight: too many weights");
+  const uint32_t total = (uint32_t)(Co * Ci * taps);
+  const FastDiv dc = make_fastdiv((uint32_t)Co), dt = make_fastdiv((uint32_t)taps);
+  const dim3 grid((total + 255) / 256);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (dtype_size(dtype) == 4)
+    hipLaunchKernelGGL((dgrad_weight_kernel<uint32_t>), grid, dim3(256), 0, s, static_cast<const uint32_t*>(w),
+                       static_cast<uint32_t*>(wt), (uint32_t)Ci, total, dc, dt);
+  else
+    hipLaunchKernelGGL((dgrad_weight_kernel<uint16_t>), grid, dim3(256), 0, s, static_cast<const uint16_t*>(w),
+                       static_cast<uint16_t*>(wt), (uint32_t)Ci, total, dc, dt);
+  return check_launch("dgrad_weight_kernel");
 }

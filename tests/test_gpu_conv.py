@@ -441,6 +441,18 @@ def test_conv_wgrad_kernel_matches_float64(case, dtype):
     assert err <= 1e-4, f"max_rel_err {err:.3g}"
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (3, 5, 3, 3), (64, 33, 3, 3, 3), (7, 130, 1, 3, 7), (256, 2, 7, 7)])
+def test_conv_dgrad_weight_is_the_flipped_transpose(shape, dtype):
+    """Exactly torch's transpose and flip, for contiguous weights and (through torch) others."""
+    from amd_tuned_torch import _native
+    w = torch.randn(*shape, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    for v in (w, w.transpose(-1, -2)):
+        want = v.transpose(0, 1).flip(list(range(2, v.dim()))).contiguous()
+        got = _native.conv_dgrad_weight(v)
+        assert got.is_contiguous() and torch.equal(got, want)
+
+
 # 3x3 planes over rows that are not 16-byte aligned: a row of one full and one partial chunk, partial
 # chunks of 1 .. 7 elements, in the first and in later column tiles, channel counts off the stage's
 # block, rows of exactly one chunk from a misaligned base
