@@ -25,6 +25,7 @@
 // LDS window would not fit.
 #include <cstring>
 
+#include "param_loads.h"
 #include "atk_common.h"
 
 namespace atk {
@@ -1216,8 +1217,7 @@ __global__ __launch_bounds__(DW_NT) void conv1d_bwd_rows_kernel(CrArgs a) {
   const bool live = row < a.rows;
   const uint32_t rr = live ? (uint32_t)row : 0u, d = rr - fdiv(rr, a.div_d) * a.D;
   float wv[KT], bv = 0.f;
-#pragma unroll
-  for (int j = 0; j < KT; ++j) wv[j] = load_param(a.w, a.wdt, (int64_t)d * a.wc + (int64_t)j * a.wk);
+  load_params<KT>(a.w, a.wdt, (int64_t)d * a.wc, a.wk, wv);
   if (SILU && a.b) bv = load_param(a.b, a.wdt, d);
   const int L = a.L, ulo = -a.sh, uhi = a.Lout - a.sh;  // g is zero outside [ulo, uhi)
   const int pend = max(L, uhi);

@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "gn_any.h"
+#include "param_loads.h"
 
 namespace atk {
 
@@ -276,8 +277,9 @@ int launch_any(const GaArgs& a, int64_t ngroups, int silu, hipStream_t s) {
 //          channels in a fixed order; one (mean, M2) record per (chunk, group);
 //   apply: every workgroup merges its sample's records itself (the first rows of x are loaded
 //          before that), then normalises its chunk.
-// [16, 128, 64, 64] bf16 with SiLU: 73 us (stock: layout copies, moments, scale, SiLU) -> 17.5 us
-// (6.5 the statistics, 2.6 TB/s; 11 the second pass, 3.0 TB/s).
+// [16, 128, 64, 64] bf16 with SiLU: 73.9 us (stock: layout copies, moments, scale, SiLU) -> 15.7 us:
+// 6.9 the statistics (2.4 TB/s), 9.0 the second pass (3.7 TB/s; 11.2 when the 16 parameters of a
+// thread were loaded one by one after the merge).
 // ---------------------------------------------------------------------------------------
 constexpr int GC_NT = 256;
 constexpr int GC_MAXG = 256;
@@ -384,7 +386,19 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_apply_kernel(GcArgs a, int la
       b[u].raw = ld16<true>(p);  // the last read of x
     }
   };
-  if (r < a.R) issue(s0 + r);
+  float gm[VEC], bt[VEC];
+  int gr[VEC];  // the group of each channel
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    gm[k] = 1.f;
+    bt[k] = 0.f;
+    gr[k] = (v * VEC + k) / a.cpg;
+  }
+  if (r < a.R) {
+    issue(s0 + r);
+    if (a.gamma) load_params<VEC>(a.gamma, a.pdt, v * VEC, 1, gm);
+    if (a.beta) load_params<VEC>(a.beta, a.pdt, v * VEC, 1, bt);
+  }
   // `lanes` lanes (a power of two, at most 64) per group merge the sample's records in a fixed order
   const int j = tid & (lanes - 1);
   for (int g = tid / lanes; g < a.G; g += GC_NT / lanes) {
@@ -424,11 +438,8 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_apply_kernel(GcArgs a, int la
   float sc[VEC], sh[VEC];
 #pragma unroll
   for (int k = 0; k < VEC; ++k) {
-    const int c = v * VEC + k, g = c / a.cpg;
-    const float gm = a.gamma ? load_param(a.gamma, a.pdt, c) : 1.f;
-    const float bt = a.beta ? load_param(a.beta, a.pdt, c) : 0.f;
-    sc[k] = g_rstd[g] * gm;
-    sh[k] = bt - g_mean[g] * sc[k];
+    sc[k] = g_rstd[gr[k]] * gm[k];
+    sh[k] = bt[k] - g_mean[gr[k]] * sc[k];
   }
   for (int64_t p0 = s0 + r; p0 < s1; p0 += (int64_t)GC_U * a.R) {
     if (p0 != s0 + r) issue(p0);
