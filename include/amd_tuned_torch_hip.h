@@ -564,6 +564,13 @@ typedef struct atk_dwconv1d_args {
 } atk_dwconv1d_args;
 int atk_dwconv1d_fwd_args(const atk_dwconv1d_args* a);
 
+typedef struct atk_causal_conv1d_update_args {
+  const void* x; void* conv_state; const void* w; const void* bias; void* y;
+  int64_t B; int64_t D; int W; int dtype; int w_dtype; int fuse_silu;
+  atk_stream_t stream;
+} atk_causal_conv1d_update_args;
+int atk_causal_conv1d_update_args_fwd(const atk_causal_conv1d_update_args* a);
+
 typedef struct atk_group_norm_args {
   const void* x; const void* gamma; const void* beta; void* y;
   int64_t N; int64_t C; int64_t S; int G; float eps; int fuse_silu;

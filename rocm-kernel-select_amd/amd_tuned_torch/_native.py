@@ -52,6 +52,7 @@ EXPORTED_SYMBOLS = (
     "atk_conv_fwd_prepacked_ex", "atk_conv_gn_onepass_workspace_bytes", "atk_conv_group_norm_fwd",
     "atk_group_norm_apply", "atk_group_norm_cl_bwd_workspace_bytes", "atk_group_norm_cl_bwd",
     "atk_dwconv1d_fwd_args", "atk_group_norm_fwd_args", "atk_conv_fwd_prepacked_args",
+    "atk_causal_conv1d_update_args_fwd",
 )
 
 
@@ -65,6 +66,13 @@ class _DwArgs(ctypes.Structure):
                 ("N", ctypes.c_int64), ("C", ctypes.c_int64), ("L", ctypes.c_int64), ("K", ctypes.c_int),
                 ("pad_left", ctypes.c_int), ("L_out", ctypes.c_int64), ("dtype", ctypes.c_int),
                 ("w_dtype", ctypes.c_int), ("fuse_silu", ctypes.c_int), ("variant", ctypes.c_int),
+                ("stream", ctypes.c_void_p)]
+
+
+class _UpdateArgs(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_void_p), ("conv_state", ctypes.c_void_p), ("w", ctypes.c_void_p),
+                ("bias", ctypes.c_void_p), ("y", ctypes.c_void_p), ("B", ctypes.c_int64), ("D", ctypes.c_int64),
+                ("W", ctypes.c_int), ("dtype", ctypes.c_int), ("w_dtype", ctypes.c_int), ("fuse_silu", ctypes.c_int),
                 ("stream", ctypes.c_void_p)]
 
 
@@ -216,7 +224,8 @@ def _declare(lib) -> None:
     lib.atk_group_norm_fwd_noalloc.argtypes = [vp, vp, vp, vp, i64, i64, i64, i32, c.c_float, i32, i32, i32,
                                                i32, vp]
     lib.atk_group_norm_fwd_noalloc.restype = i32
-    for name in ("atk_dwconv1d_fwd_args", "atk_group_norm_fwd_args", "atk_conv_fwd_prepacked_args"):
+    for name in ("atk_dwconv1d_fwd_args", "atk_group_norm_fwd_args", "atk_conv_fwd_prepacked_args",
+                 "atk_causal_conv1d_update_args_fwd"):
         getattr(lib, name).argtypes = [vp]
         getattr(lib, name).restype = i32
 
@@ -462,10 +471,11 @@ def causal_conv1d_update(x: torch.Tensor, conv_state: torch.Tensor, weight: torc
         raise RuntimeError("causal_conv1d_update expects x [B, D], conv_state [B, D, W], weight [D, W]")
     B, D = x.shape
     W = weight.shape[1]
-    if tuple(conv_state.shape) != (B, D, W) or weight.shape[0] != D:
+    if conv_state.shape != (B, D, W) or weight.shape[0] != D:
         raise RuntimeError("causal_conv1d_update: conv_state must be [B, D, W] and weight [D, W]")
-    if x.dtype not in _DTYPE_CODE or conv_state.dtype != x.dtype or weight.dtype not in (x.dtype, torch.float32) \
-            or (bias is not None and bias.dtype != weight.dtype):
+    dt, wdt = x.dtype, weight.dtype
+    if dt not in _DTYPE_CODE or conv_state.dtype != dt or wdt not in (dt, torch.float32) \
+            or (bias is not None and bias.dtype != wdt):
         raise RuntimeError("causal_conv1d_update: x and conv_state must share a dtype; weight and bias that "
                            "dtype or fp32")
     if not conv_state.is_contiguous():
@@ -474,10 +484,15 @@ def causal_conv1d_update(x: torch.Tensor, conv_state: torch.Tensor, weight: torc
     weight = weight.contiguous()
     bias = bias.contiguous() if bias is not None else None
     y = torch.empty_like(x)
-    rc = lib().atk_causal_conv1d_update(_ptr(x), _ptr(conv_state), _ptr(weight), _ptr(bias), _ptr(y), B, D, W,
-                                        _DTYPE_CODE[x.dtype], _DTYPE_CODE[weight.dtype], int(bool(silu)),
-                                        _stream(x))
-    _check(rc, "causal_conv1d_update")
+    blk = _block("upd", _UpdateArgs)
+    a = blk[0]
+    key = (B, D, W, dt, wdt, silu)
+    if blk[2] != key:
+        a.B, a.D, a.W, a.dtype, a.w_dtype, a.fuse_silu = B, D, W, _DTYPE_CODE[dt], _DTYPE_CODE[wdt], int(bool(silu))
+        blk[2] = key
+    a.x, a.conv_state, a.w, a.bias = x.data_ptr(), conv_state.data_ptr(), weight.data_ptr(), _ptr(bias)
+    a.y, a.stream = y.data_ptr(), _stream(x)
+    _check(lib().atk_causal_conv1d_update_args_fwd(blk[1]), "causal_conv1d_update")
     return y
 
 

@@ -37,7 +37,7 @@ def _channel_last(x: torch.Tensor) -> bool:
 def _kernel_weight(weight: torch.Tensor, x: torch.Tensor, bias):
     """The weights (and bias) as the kernels take them: fp32, or x's dtype."""
     w = weight if weight.dtype in (torch.float32, x.dtype) else weight.float()
-    return w, (bias.to(w.dtype) if bias is not None else None)
+    return w, (bias if bias is None or bias.dtype == w.dtype else bias.to(w.dtype))
 
 
 def _forward(x, weight, bias, seq_idx, initial_states, final_states_out, silu: bool):
@@ -117,6 +117,37 @@ def _backward(x, weight, bias, dout, seq_idx, initial_states, dfinal, silu: bool
     return dx, dw.to(weight.dtype), (db.to(bias.dtype) if bias is not None else None), dinit
 
 
+def _checked(x, weight, bias, activation):
+    """(x, bias) as the kernels take them, after the interface's argument checks."""
+    if activation not in (None, "silu", "swish"):
+        raise NotImplementedError("activation must be None, silu, or swish")
+    if x.dim() != 3 or weight.dim() != 2 or weight.shape[0] != x.shape[1]:
+        raise RuntimeError("causal_conv1d_fn: expects x (batch, dim, seqlen), weight (dim, width)")
+    if not 2 <= weight.shape[1] <= 4:
+        raise RuntimeError("causal_conv1d only supports width between 2 and 4")
+    if x.stride(2) != 1 and x.stride(1) != 1:
+        x = x.contiguous()
+    return x, (bias.contiguous() if bias is not None else None)
+
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _no_autograd(x, weight, bias) -> bool:
+    """True when no part of autograd can be watching: plain tensors, no gradient wanted, and no
+    functorch transform, forward-mode level, torch-function or dispatch mode, or trace active.  The
+    autograd Function then adds nothing but its own cost (about 4 us, a third of a small call)."""
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad
+                                    or (bias is not None and bias.requires_grad)):
+        return False
+    return (type(x) in _PLAIN and type(weight) in _PLAIN and (bias is None or type(bias) in _PLAIN)
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+
+
 class CausalConv1dFn(torch.autograd.Function):
     """The reference's CausalConv1dFn (causal_conv1d_interface.py:10-98): same argument
     checks, same saved tensors, same gradient outputs."""
@@ -124,15 +155,7 @@ class CausalConv1dFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias=None, seq_idx=None, initial_states=None, return_final_states=False,
                 final_states_out=None, activation=None):
-        if activation not in (None, "silu", "swish"):
-            raise NotImplementedError("activation must be None, silu, or swish")
-        if x.dim() != 3 or weight.dim() != 2 or weight.shape[0] != x.shape[1]:
-            raise RuntimeError("causal_conv1d_fn: expects x (batch, dim, seqlen), weight (dim, width)")
-        if not 2 <= weight.shape[1] <= 4:
-            raise RuntimeError("causal_conv1d only supports width between 2 and 4")
-        if x.stride(2) != 1 and x.stride(1) != 1:
-            x = x.contiguous()
-        bias = bias.contiguous() if bias is not None else None
+        x, bias = _checked(x, weight, bias, activation)
         if seq_idx is not None:
             assert initial_states is None, "initial_states must be None if seq_idx is not None"
             assert not return_final_states, "If seq_idx is not None, we don't return final_states_out"
@@ -174,6 +197,9 @@ def causal_conv1d_fn(x, weight, bias=None, seq_idx=None, initial_states=None,
     """x (batch, dim, seqlen), weight (dim, width), bias (dim,), seq_idx int32 (batch, seqlen),
     initial_states / final_states_out (batch, dim, width - 1); returns out, or (out,
     final_states) with return_final_states (causal_conv1d_interface.py:100-130)."""
+    if seq_idx is None and initial_states is None and not return_final_states and _no_autograd(x, weight, bias):
+        x, bias = _checked(x, weight, bias, activation)
+        return _forward(x, weight, bias, None, None, None, activation is not None)
     return CausalConv1dFn.apply(x, weight, bias, seq_idx, initial_states, return_final_states,
                                 final_states_out, activation)
 

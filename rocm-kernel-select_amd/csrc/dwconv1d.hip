@@ -1605,3 +1605,9 @@ extern "C" int atk_dwconv1d_fwd_args(const atk_dwconv1d_args* a) {
   return atk_dwconv1d_fwd(a->x, a->w, a->bias, a->y, a->N, a->C, a->L, a->K, a->pad_left, a->L_out, a->dtype,
                           a->w_dtype, a->fuse_silu, a->variant, a->stream);
 }
+
+extern "C" int atk_causal_conv1d_update_args_fwd(const atk_causal_conv1d_update_args* a) {
+  if (!a) return atk::fail(ATK_EINVAL, "causal_conv1d_update: null argument block");
+  return atk_causal_conv1d_update(a->x, a->conv_state, a->w, a->bias, a->y, a->B, a->D, a->W, a->dtype, a->w_dtype,
+                                  a->fuse_silu, a->stream);
+}

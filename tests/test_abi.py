@@ -217,3 +217,19 @@ def test_argument_blocks_validate_like_their_entry_points(nat):
         c = nat._ConvArgs(None, None, 0, None, None, *geom, dt, v, None, 0, None)
         assert lib.atk_conv_fwd_prepacked_args(ctypes.addressof(c)) == \
             lib.atk_conv_fwd_prepacked(None, None, 0, None, None, *geom, dt, v, None, 0, None)
+
+
+def test_update_argument_block_layout_matches_the_header(nat, tmp_path):
+    """As above for atk_causal_conv1d_update_args; a null block is refused."""
+    cls, cname = nat._UpdateArgs, "atk_causal_conv1d_update_args"
+    fields = [f for f, _ in cls._fields_]
+    src = tmp_path / "layout.c"
+    src.write_text("\n".join(
+        ["#include <stdio.h>", "#include <stddef.h>", f'#include "{HEADER}"', "int main(void) {",
+         f'  printf("%zu\\n", sizeof({cname}));']
+        + [f'  printf("%zu\\n", offsetof({cname}, {f}));' for f in fields] + ["  return 0;", "}"]))
+    exe = tmp_path / "layout"
+    subprocess.run(["gcc", "-O0", str(src), "-o", str(exe)], check=True)
+    got = subprocess.run([str(exe)], check=True, stdout=subprocess.PIPE, text=True).stdout.split()
+    assert [int(g) for g in got] == [ctypes.sizeof(cls)] + [getattr(cls, f).offset for f in fields]
+    assert nat.lib().atk_causal_conv1d_update_args_fwd(None) == nat.ATK_EINVAL

@@ -75,3 +75,63 @@ def test_ref_statements_agree_with_each_other():
     state = torch.cat([torch.zeros(2, 16, 1, dtype=torch.float64), x[..., -4:-1]], dim=-1)
     step = cc.causal_conv1d_update_ref(x[..., -1], state, w, b, activation="silu")
     torch.testing.assert_close(step, cc.causal_conv1d_ref(x, w, b, activation="silu")[..., -1])
+
+
+def test_direct_call_only_where_no_part_of_autograd_watches():
+    """causal_conv1d_fn leaves the autograd Function out only for plain tensors that want no
+    gradient, outside functorch transforms, forward-mode levels, modes and traces."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from amd_tuned_torch import causal_conv1d as cc
+    x, w, b = torch.zeros(1, 4, 8), torch.zeros(4, 3), torch.zeros(4)
+    assert cc._no_autograd(x, w, b) and cc._no_autograd(x, w, None)
+    for k in range(3):
+        leaves = [t.clone() for t in (x, w, b)]
+        leaves[k].requires_grad_()
+        assert not cc._no_autograd(*leaves)
+        with torch.no_grad():
+            assert cc._no_autograd(*leaves)
+    assert cc._no_autograd(x, torch.nn.Parameter(w, requires_grad=False), b)
+
+    class Sub(torch.Tensor):
+        pass
+    assert not cc._no_autograd(x.as_subclass(Sub), w, b)
+    with torch.autograd.forward_ad.dual_level():
+        assert not cc._no_autograd(x, w, b)
+    seen = []
+    torch.func.vmap(lambda t: seen.append(cc._no_autograd(x, w, b)) or t)(torch.zeros(2))
+    assert seen == [False]
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    with Function():
+        assert not cc._no_autograd(x, w, b)
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    with Dispatch():
+        assert not cc._no_autograd(x, w, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("channel_last", [False, True])
+def test_direct_call_equals_the_autograd_function(channel_last):
+    """The same bits, layout and argument errors with and without the Function."""
+    from amd_tuned_torch import causal_conv1d as cc
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn(2, 16, 37, generator=g).to(torch.bfloat16).cuda()
+    if channel_last:
+        x = x.transpose(1, 2).contiguous().transpose(1, 2)
+    w, b = torch.randn(16, 4, generator=g).cuda(), torch.randn(16, generator=g).cuda()
+    for act in (None, "silu"):
+        a = cc.causal_conv1d_fn(x, w, b, activation=act)
+        r = cc.causal_conv1d_fn(x, w.clone().requires_grad_(), b, activation=act)
+        assert r.requires_grad and not a.requires_grad
+        assert torch.equal(a, r) and a.stride() == r.stride()
+    with pytest.raises(NotImplementedError):
+        cc.causal_conv1d_fn(x, w, b, activation="relu")
+    with pytest.raises(RuntimeError):
+        cc.causal_conv1d_fn(x, torch.zeros(16, 5, device="cuda"), None)
