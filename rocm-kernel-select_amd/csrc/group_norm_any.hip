@@ -277,8 +277,9 @@ int launch_any(const GaArgs& a, int64_t ngroups, int silu, hipStream_t s) {
 //          channels in a fixed order; one (mean, M2) record per (chunk, group);
 //   apply: every workgroup merges its sample's records itself (the first rows of x are loaded
 //          before that), then normalises its chunk.
-// [16, 128, 64, 64] bf16 with SiLU: 73.9 us (stock: layout copies, moments, scale, SiLU) -> 15.7 us:
-// 6.9 the statistics (2.4 TB/s), 9.0 the second pass (3.7 TB/s; 11.2 when the 16 parameters of a
+// [16, 128, 64, 64] bf16 with SiLU: 73.9 us (stock: layout copies, moments, scale, SiLU) -> 15.0 us:
+// 6.4 the statistics (2.6 TB/s; 6.9 with the shifts waited for before the first rows were
+// requested), 9.1 the second pass (3.7 TB/s; 11.2 when the 16 parameters of a
 // thread were loaded one by one after the merge).
 // ---------------------------------------------------------------------------------------
 constexpr int GC_NT = 256;
@@ -299,12 +300,18 @@ struct GcArgs {
   int pdt;
 };
 
-// Chunks of at least one batch of rows in flight per thread (GC_U for every thread row of a 16-bit
-// tensor), about two workgroups per CU, at most 256 records a group.
+// A chunk is one batch of rows in flight per thread (GC_U for every thread row of a 16-bit tensor):
+// rounded down, the few rows over a batch cost a second round trip ([1, 128, 37, 53] bf16 11.8 us,
+// rounded up 10.5).  A quarter of that where it leaves under 64 workgroups ([16, 96, 17, 19] 10.4
+// -> 9.6 us).  At most two workgroups per CU, the 64 records a group that 8 lanes load at once
+// ([4, 128, 128, 128] 128 chunks 18.2 us, 64 chunks 15.4), and more only while a CU is without a
+// workgroup ([1, 128, 256, 256] 64 chunks 30.1 us, 256 chunks 21.0).
 int gc_chunks(int64_t N, int64_t C, int64_t S) {
   const int64_t batch = std::max<int64_t>(1, GC_NT / std::max<int64_t>(1, C / 8)) * GC_U;
-  const int64_t most = std::max<int64_t>(1, 512 / std::max<int64_t>(1, N));
-  const int64_t ch = std::max<int64_t>(1, std::min<int64_t>({S / batch, most, 256}));
+  const int64_t n = std::max<int64_t>(1, N);
+  int64_t ch = (S + batch - 1) / batch;
+  if (n * ch < 64) ch = std::min<int64_t>((S * 4 + batch - 1) / batch, std::max<int64_t>(ch, 64));
+  ch = std::max<int64_t>(1, std::min<int64_t>(ch, std::max<int64_t>(256 / n, std::min<int64_t>(512 / n, 64))));
   const int64_t rows = (S + ch - 1) / ch;
   return (int)((S + rows - 1) / rows);
 }
@@ -318,17 +325,31 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_stats_kernel(GcArgs a) {
   const int64_t s0 = (int64_t)ch * a.rows, s1 = min(s0 + a.rows, a.S);
   const T* __restrict__ xn = static_cast<const T*>(a.x) + (int64_t)n * a.S * a.C;
   if (r < a.R) {
-    float K[VEC], a1[VEC], a2[VEC];
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      K[k] = to_f32(xn[s0 * a.C + (v * VEC + k) / a.cpg * a.cpg]);
-      a1[k] = a2[k] = 0.f;
-    }
-    for (int64_t p0 = s0 + r; p0 < s1; p0 += (int64_t)GC_U * a.R) {
-      Vec16<T> b[GC_U];
+    Vec16<T> b[GC_U];
+    auto issue = [&](int64_t p0) {
 #pragma unroll
       for (int u = 0; u < GC_U; ++u)
         b[u].raw = *reinterpret_cast<const uint4*>(xn + min(p0 + (int64_t)u * a.R, s1 - 1) * a.C + v * VEC);
+    };
+    issue(s0 + r);  // in flight together with the shifts
+    float K[VEC], a1[VEC], a2[VEC];
+    const T* xk = xn + s0 * a.C;
+    int g0 = v * VEC / a.cpg * a.cpg, left = g0 + a.cpg - v * VEC;  // the group's first channel, channels left in it
+    T kv[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      kv[k] = xk[g0];
+      const bool next = --left == 0;
+      g0 += next ? a.cpg : 0;
+      left = next ? a.cpg : left;
+    }
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {
+      K[k] = to_f32(kv[k]);
+      a1[k] = a2[k] = 0.f;
+    }
+    for (int64_t p0 = s0 + r; p0 < s1; p0 += (int64_t)GC_U * a.R) {
+      if (p0 != s0 + r) issue(p0);
 #pragma unroll
       for (int u = 0; u < GC_U; ++u) {
         const bool ok = p0 + (int64_t)u * a.R < s1;
@@ -349,6 +370,7 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_stats_kernel(GcArgs a) {
   __syncthreads();
   for (int c = tid; c < a.C; c += GC_NT) {  // over the thread rows, into row 0
     float t1 = l1[c], t2 = l2[c];
+#pragma unroll 4
     for (int q = 1; q < a.R; ++q) {
       t1 += l1[q * a.C + c];
       t2 += l2[q * a.C + c];
@@ -387,12 +409,10 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_apply_kernel(GcArgs a, int la
     }
   };
   float gm[VEC], bt[VEC];
-  int gr[VEC];  // the group of each channel
 #pragma unroll
   for (int k = 0; k < VEC; ++k) {
     gm[k] = 1.f;
     bt[k] = 0.f;
-    gr[k] = (v * VEC + k) / a.cpg;
   }
   if (r < a.R) {
     issue(s0 + r);
@@ -436,10 +456,14 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_apply_kernel(GcArgs a, int la
   __syncthreads();
   if (r >= a.R) return;
   float sc[VEC], sh[VEC];
+  int g = v * VEC / a.cpg, left = (g + 1) * a.cpg - v * VEC;  // the channel's group, channels left in it
 #pragma unroll
   for (int k = 0; k < VEC; ++k) {
-    sc[k] = g_rstd[gr[k]] * gm[k];
-    sh[k] = bt[k] - g_mean[gr[k]] * sc[k];
+    sc[k] = g_rstd[g] * gm[k];
+    sh[k] = bt[k] - g_mean[g] * sc[k];
+    const bool next = --left == 0;
+    g = min(g + next, a.G - 1);
+    left = next ? a.cpg : left;
   }
   for (int64_t p0 = s0 + r; p0 < s1; p0 += (int64_t)GC_U * a.R) {
     if (p0 != s0 + r) issue(p0);

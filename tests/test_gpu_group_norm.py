@@ -561,6 +561,10 @@ CL_ANY_SHAPES = [
     ((2, 48, 1, 1), 1),
     ((1, 256, 3, 17, 19), 256),
     ((1, 1000, 13, 4), 4),
+    # chunks of a quarter batch, more records than 8 lanes load at once, the cap of a large batch
+    ((1, 128, 37, 53), 32),
+    ((1, 128, 130, 131), 32),
+    ((65, 64, 33, 3), 32),
 ]
 
 
