@@ -956,7 +956,24 @@ __global__ __launch_bounds__(GN_TP_NT) void gn_bwd_rows_kernel(GnBwdArgs a) {
   const int64_t r = blockIdx.x;
   const T* __restrict__ xr = static_cast<const T*>(a.x) + r * a.S;
   const T* __restrict__ gr = static_cast<const T*>(a.dy) + r * a.S;
-  const float K = to_f32(xr[0]);
+  // RAG: the mean of the row's first vector, nearer to the row's mean than one value, and each
+  // vector summed by itself first.  Both only for accuracy: fp32 dgamma over [3,448,33,54] against
+  // 64 bits 1.3e-7; with the one value and one running sum 1.8e-7
+  float K;
+  if constexpr (RAG) {
+    Vec16<T> f;
+    f.raw = gn_ld16u(xr);
+    float t[VEC];
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) t[k] = to_f32(f.e[k]) * (1.f / VEC);
+#pragma unroll
+    for (int h = VEC / 2; h; h >>= 1)
+#pragma unroll
+      for (int k = 0; k < h; ++k) t[k] += t[k + h];
+    K = t[0];
+  } else {
+    K = to_f32(xr[0]);
+  }
   float s1 = 0.f, s2 = 0.f, sa = 0.f, sb = 0.f;
   // U vectors of x and of dy in flight per thread (branch-free buffer loads; vectors
   // past the row read zero and are masked out of the sums)
@@ -982,15 +999,24 @@ __global__ __launch_bounds__(GN_TP_NT) void gn_bwd_rows_kernel(GnBwdArgs a) {
       if constexpr (RAG) {
         const int64_t e = e0 + (int64_t)u * GN_TP_NT * VEC;
         const int skip = e >= a.S ? VEC : (int)max(e - (a.S - VEC), (int64_t)0);
+        float d[VEC], g[VEC];
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
-          const float d = k >= skip ? to_f32(xv[u].e[k]) - K : 0.f;
-          const float g = k >= skip ? to_f32(gv[u].e[k]) : 0.f;
-          s1 += d;
-          s2 = fmaf(d, d, s2);
-          sa += g;
-          sb = fmaf(g, d, sb);
+          d[k] = k >= skip ? to_f32(xv[u].e[k]) - K : 0.f;
+          g[k] = k >= skip ? to_f32(gv[u].e[k]) : 0.f;
         }
+        float v1 = 0.f, v2 = 0.f, va = 0.f, vb = 0.f;
+#pragma unroll
+        for (int k = 0; k < VEC; k += 2) {
+          v1 += d[k] + d[k + 1];
+          v2 += fmaf(d[k], d[k], d[k + 1] * d[k + 1]);
+          va += g[k] + g[k + 1];
+          vb += fmaf(g[k], d[k], g[k + 1] * d[k + 1]);
+        }
+        s1 += v1;
+        s2 += v2;
+        sa += va;
+        sb += vb;
         continue;
       }
       const float m = (e0 + (int64_t)u * GN_TP_NT * VEC < a.S) ? 1.f : 0.f;
