@@ -438,17 +438,25 @@ def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups,
     return dw.view(weight.shape).to(weight.dtype), None if db is None else db.to(weight.dtype)
 
 
+def _graph_wanted(*tensors) -> bool:
+    """True when the gradients being computed are to be differentiated again (create_graph=True):
+    the native backward kernels record nothing, so they must not serve the call."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+
+
 def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
     """(dx, dw, db) of a patched conv for `needs` = [dx, dw, db] wanted:
     * dx of a stride-1, dilation-1, groups-1 conv through `fwd` (the accelerated forward) on dy
       with transposed, flipped weights;
     * dw of a 'same' 3x3(x3) conv in a 16-bit type through the native wgrad kernel, db with it;
     * db alone as a reduction of dy once every other gradient is native;
-    * whatever is left through aten.convolution_backward, the op autograd uses unpatched."""
+    * whatever is left, and everything that is to be differentiated again, through
+      aten.convolution_backward, the op autograd uses unpatched."""
     stride, padding, dilation, groups, nd = conf
     needs = list(needs)
     gi = gw = gb = None
-    if needs[0] and input.is_cuda:
+    native = input.is_cuda and not _graph_wanted(grad_output, input, weight)
+    if needs[0] and native:
         pad_t = _dgrad_padding(weight, stride, padding, dilation, groups, nd)
         if pad_t is not None:
             gi = _dgrad_via_forward(grad_output, weight.detach(), pad_t, nd, fwd)
@@ -456,7 +464,7 @@ def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
                 needs[0] = False
             else:
                 gi = None
-    if needs[1] and input.is_cuda:
+    if needs[1] and native:
         got = _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd, needs[2])
         if got is not None:
             gw, gb = got
@@ -738,8 +746,15 @@ def _group_norm_grads(grad_output, input, num_groups, weight, eps, needs):
     backward kernels for contiguous or channels-last GPU input (channels-last first on the
     channels-last kernels, else through NC[S] copies made by the native transpose, dx coming
     back in the input's layout; dgamma / dbeta in fp32), the textbook torch-op backward
-    otherwise (dgamma / dbeta in the parameter dtypes).  Entries not asked for are None."""
+    otherwise (dgamma / dbeta in the parameter dtypes).  Gradients that are to be differentiated
+    again take the torch ops too, 16-bit ones on the GPU in fp32, as the kernels compute.
+    Entries not asked for are None."""
     cl = _channels_last(input)
+    if input.is_cuda and _graph_wanted(grad_output, input, weight):
+        acc = torch.promote_types(input.dtype, torch.float32)
+        gx, gw, gb = _group_norm_backward(grad_output.to(acc).contiguous(), input.to(acc), num_groups,
+                                          None if weight is None else weight.to(acc), eps, needs)
+        return None if gx is None else gx.to(input.dtype), gw, gb
     if input.is_cuda and cl and _native.available():
         try:  # straight on the channels-last layout
             fmt = torch.channels_last if input.dim() == 4 else torch.channels_last_3d
