@@ -270,11 +270,14 @@ int launch_any(const GaArgs& a, int64_t ngroups, int silu, hipStream_t s) {
 // ---------------------------------------------------------------------------------------
 // Channels-last, any channels per group.  A thread owns one 16-byte channel vector (column) on
 // every R-th position of a chunk; 256 / columns rows of threads, the rest of the 256 idle.  A
-// column may span several groups and a group several columns, so the sums are kept per channel,
-// all about one shift per group (the group's first value in the chunk: one of its values, so
-// the cancellation is bounded), which makes them plain sums across threads and channels:
-//   stats: per-channel sums of the chunk, added over the thread rows and then over the group's
-//          channels in a fixed order; one (mean, M2) record per (chunk, group);
+// column may span several groups and a group several columns, so the moments are kept per channel:
+//   stats: each thread sums its positions of a channel about the mean of its first four, and the
+//          threads' (mean, M2) are merged exactly, over the thread rows and then over the group's
+//          channels, in a fixed order; one (mean, M2) record per (chunk, group).  A value far
+//          from the rest thus cancels against the n positions of its own thread at a quarter of
+//          its size, which bounds M2's relative error by about n / 16 * 2^-24 (one shift for a
+//          chunk and group let it reach rows * channels * 2^-24: 3e-4 in rstd over
+//          [1, 96, 96, 96], G = 1 with one value of 1e3, now 1e-7).
 //   apply: every workgroup merges its sample's records itself (the first rows of x are loaded
 //          before that), then normalises its chunk.
 // [16, 128, 64, 64] bf16 with SiLU: 73.9 us (stock: layout copies, moments, scale, SiLU) -> 15.0 us:
@@ -296,6 +299,7 @@ struct GcArgs {
   int N, C, G, cpg, NCH;
   int rows;      // positions per chunk
   int cols, R;   // channel vectors, thread rows
+  FastDiv div_r;
   float eps;
   int pdt;
 };
@@ -316,14 +320,24 @@ int gc_chunks(int64_t N, int64_t C, int64_t S) {
   return (int)((S + rows - 1) / rows);
 }
 
+// Mean of the first four of p[0], p[stride], .. (n of them; the last stands in for those missing): the
+// shift of a merge, such that one far value among them weighs a quarter.
+__device__ __forceinline__ float mean4(const float* p, int stride, int n) {
+  const float t0 = p[0], t1 = p[min(1, n - 1) * stride], t2 = p[min(2, n - 1) * stride], t3 = p[min(3, n - 1) * stride];
+  return 0.25f * ((t0 + t1) + (t2 + t3));
+}
+
 template <typename T>
-__global__ __launch_bounds__(GC_NT) void gn_cl_any_stats_kernel(GcArgs a) {
+__global__ __launch_bounds__(GC_NT) void gn_cl_any_stats_kernel(GcArgs a, int lanes) {
   constexpr int VEC = Vec16<T>::N;
-  __shared__ float l1[GC_NT * VEC], l2[GC_NT * VEC];
+  __shared__ __align__(16) float l1[GC_NT * VEC], l2[GC_NT * VEC];
   const int tid = threadIdx.x, r = tid / a.cols, v = tid - r * a.cols;
   const int n = blockIdx.x / a.NCH, ch = blockIdx.x - n * a.NCH;
   const int64_t s0 = (int64_t)ch * a.rows, s1 = min(s0 + a.rows, a.S);
   const T* __restrict__ xn = static_cast<const T*>(a.x) + (int64_t)n * a.S * a.C;
+  // thread row q holds per + (q < more) of the chunk's len positions
+  const int len = (int)(s1 - s0), per = (int)fdiv((uint32_t)len, a.div_r), more = len - per * a.R;
+  const float wl = (float)per, wm = (float)(per + 1);
   if (r < a.R) {
     Vec16<T> b[GC_U];
     auto issue = [&](int64_t p0) {
@@ -331,63 +345,94 @@ __global__ __launch_bounds__(GC_NT) void gn_cl_any_stats_kernel(GcArgs a) {
       for (int u = 0; u < GC_U; ++u)
         b[u].raw = *reinterpret_cast<const uint4*>(xn + min(p0 + (int64_t)u * a.R, s1 - 1) * a.C + v * VEC);
     };
-    issue(s0 + r);  // in flight together with the shifts
     float K[VEC], a1[VEC], a2[VEC];
-    const T* xk = xn + s0 * a.C;
-    int g0 = v * VEC / a.cpg * a.cpg, left = g0 + a.cpg - v * VEC;  // the group's first channel, channels left in it
-    T kv[VEC];
+    auto add = [&](int64_t p0) {
+      // all of a batch is requested before any of it is used (else it is waited for in turn)
 #pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      kv[k] = xk[g0];
-      const bool next = --left == 0;
-      g0 += next ? a.cpg : 0;
-      left = next ? a.cpg : left;
-    }
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      K[k] = to_f32(kv[k]);
-      a1[k] = a2[k] = 0.f;
-    }
-    for (int64_t p0 = s0 + r; p0 < s1; p0 += (int64_t)GC_U * a.R) {
-      if (p0 != s0 + r) issue(p0);
+      for (int u = 0; u < GC_U; ++u)
+        asm volatile("" : : "v"(b[u].raw.x), "v"(b[u].raw.y), "v"(b[u].raw.z), "v"(b[u].raw.w));
 #pragma unroll
       for (int u = 0; u < GC_U; ++u) {
-        const bool ok = p0 + (int64_t)u * a.R < s1;
+        if (p0 + (int64_t)u * a.R >= s1) break;
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
-          const float d = ok ? to_f32(b[u].e[k]) - K[k] : 0.f;
+          const float d = to_f32(b[u].e[k]) - K[k];
           a1[k] += d;
           a2[k] = fmaf(d, d, a2[k]);
         }
       }
+    };
+    int64_t p0 = s0 + r;
+    issue(p0);
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) {  // (positions past the chunk repeat its last one: any value is a shift)
+      K[k] = 0.25f * ((to_f32(b[0].e[k]) + to_f32(b[1].e[k])) + (to_f32(b[2].e[k]) + to_f32(b[3].e[k])));
+      a1[k] = a2[k] = 0.f;
     }
+    add(p0);
+    while ((p0 += (int64_t)GC_U * a.R) < s1) {
+      issue(p0);
+      add(p0);
+    }
+    const int cnt = per + (r < more);
+    const float inv = cnt ? __builtin_amdgcn_rcpf((float)cnt) : 0.f;
+    float4* o1 = reinterpret_cast<float4*>(l1 + r * a.C + v * VEC);
+    float4* o2 = reinterpret_cast<float4*>(l2 + r * a.C + v * VEC);
 #pragma unroll
     for (int k = 0; k < VEC; ++k) {
-      l1[r * a.C + v * VEC + k] = a1[k];
-      l2[r * a.C + v * VEC + k] = a2[k];
+      const float q = a1[k] * inv;
+      a2[k] = fmaxf(fmaf(-a1[k], q, a2[k]), 0.f);
+      a1[k] = cnt ? K[k] + q : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < VEC; k += 4) {
+      o1[k / 4] = make_float4(a1[k], a1[k + 1], a1[k + 2], a1[k + 3]);
+      o2[k / 4] = make_float4(a2[k], a2[k + 1], a2[k + 2], a2[k + 3]);
     }
   }
   __syncthreads();
-  for (int c = tid; c < a.C; c += GC_NT) {  // over the thread rows, into row 0
-    float t1 = l1[c], t2 = l2[c];
+  const float inv_len = __builtin_amdgcn_rcpf((float)len);
+  for (int c = 2 * tid; c < a.C; c += 2 * GC_NT) {  // over the thread rows, two channels a thread, into row 0
+    const float m0 = mean4(l1 + c, a.C, a.R), n0 = mean4(l1 + c + 1, a.C, a.R);
+    float t1 = 0.f, t2 = 0.f, u1 = 0.f, u2 = 0.f;
 #pragma unroll 4
-    for (int q = 1; q < a.R; ++q) {
-      t1 += l1[q * a.C + c];
-      t2 += l2[q * a.C + c];
+    for (int q = 0; q < a.R; ++q) {
+      const float2 m = *reinterpret_cast<const float2*>(l1 + q * a.C + c);
+      const float2 s = *reinterpret_cast<const float2*>(l2 + q * a.C + c);
+      const float w = q < more ? wm : wl, d = m.x - m0, e = m.y - n0;
+      t1 = fmaf(w, d, t1);
+      u1 = fmaf(w, e, u1);
+      t2 += fmaf(w * d, d, s.x);
+      u2 += fmaf(w * e, e, s.y);
     }
-    l1[c] = t1;
-    l2[c] = t2;
+    const float q = t1 * inv_len, h = u1 * inv_len;
+    *reinterpret_cast<float2*>(l1 + c) = make_float2(m0 + q, n0 + h);
+    *reinterpret_cast<float2*>(l2 + c) = make_float2(fmaxf(fmaf(-t1, q, t2), 0.f), fmaxf(fmaf(-u1, h, u2), 0.f));
   }
   __syncthreads();
-  if (tid < a.G) {
-    float t1 = 0.f, t2 = 0.f;
-    for (int j = 0; j < a.cpg; ++j) {
-      t1 += l1[tid * a.cpg + j];
-      t2 += l2[tid * a.cpg + j];
+  // `lanes` lanes (a power of two) per group, over its channels
+  const int j = tid & (lanes - 1), g = tid / lanes;
+  if (g < a.G) {
+    const float* gm = l1 + g * a.cpg;
+    const float* gq = l2 + g * a.cpg;
+    const float m0 = mean4(gm, 1, a.cpg);
+    float t1 = 0.f, t2 = 0.f, t3 = 0.f;
+#pragma unroll 4
+    for (int i = j; i < a.cpg; i += lanes) {
+      const float d = gm[i] - m0;
+      t1 += d;
+      t2 = fmaf(d, d, t2);
+      t3 += gq[i];
     }
-    const float q = t1 / ((float)(s1 - s0) * (float)a.cpg);
-    const float K = to_f32(xn[s0 * a.C + tid * a.cpg]);
-    a.part[((int64_t)n * a.NCH + ch) * a.G + tid] = make_float2(K + q, fmaxf(fmaf(-t1, q, t2), 0.f));
+    for (int o = lanes >> 1; o; o >>= 1) {
+      t1 += __shfl_xor(t1, o, 64);
+      t2 += __shfl_xor(t2, o, 64);
+      t3 += __shfl_xor(t3, o, 64);
+    }
+    const float q = t1 * __builtin_amdgcn_rcpf((float)a.cpg);
+    if (j == 0)
+      a.part[((int64_t)n * a.NCH + ch) * a.G + g] =
+          make_float2(m0 + q, fmaf((float)len, fmaxf(fmaf(-t1, q, t2), 0.f), t3));
   }
 }
 
@@ -485,10 +530,12 @@ template <typename T>
 int launch_cl_any(GcArgs a, int silu, hipStream_t s) {
   a.cols = a.C / (16 / (int)sizeof(T));
   a.R = GC_NT / a.cols;
+  a.div_r = make_fastdiv((uint32_t)a.R);
   int lanes = 64;
   while (lanes > 1 && lanes * a.G > GC_NT) lanes >>= 1;
   const dim3 grid((unsigned)((int64_t)a.N * a.NCH));
-  hipLaunchKernelGGL((gn_cl_any_stats_kernel<T>), grid, dim3(GC_NT), 0, s, a);
+  // (a few channels are summed faster than lanes are merged)
+  hipLaunchKernelGGL((gn_cl_any_stats_kernel<T>), grid, dim3(GC_NT), 0, s, a, a.cpg >= 32 ? lanes : 1);
   const int rc = check_launch("gn_cl_any_stats_kernel");
   if (rc) return rc;
   if (silu) hipLaunchKernelGGL((gn_cl_any_apply_kernel<T, true>), grid, dim3(GC_NT), 0, s, a, lanes);

@@ -585,6 +585,26 @@ def test_group_norm_channels_last_any_channels(dev, case, dtype):
         _check(y.cpu().contiguous(), x, G, gm, bt, 1e-5, silu=silu)
 
 
+@pytest.mark.parametrize("far", [30.0, 1e3, 1e4])
+@pytest.mark.parametrize("case", [((1, 96, 96, 96), 1), ((2, 320, 32, 32), 32), ((1, 192, 37, 53), 32)],
+                         ids=lambda s: "x".join(map(str, s[0])) + f"_g{s[1]}")
+def test_group_norm_channels_last_far_value(dev, case, far):
+    """One value per group, the first that a workgroup meets, `far` times the spread from the
+    rest.  The error of the other values relative to their own size is that of rstd: a far value
+    cancels at a quarter of its size against a thread's at most 16 positions, 2^-24 in M2, and
+    the merges over thread rows, channels and chunks and the store add about 16 roundings: 1e-6."""
+    shape, G = case
+    nat = _native()
+    x = torch.randn(*shape, generator=torch.Generator().manual_seed(G))
+    x.view(shape[0], G, shape[1] // G, -1)[:, :, 0, 0] = far
+    ref = torch.as_tensor(O.group_norm(x, G, None, None, 1e-5)).view(shape[0], G, shape[1] // G, -1)
+    y = nat.group_norm_cl(x.to(dev).contiguous(memory_format=torch.channels_last), G, None, None, 1e-5)
+    y = y.cpu().contiguous().double().view_as(ref)
+    assert (y[:, :, 0, 0] / ref[:, :, 0, 0] - 1).abs().max().item() <= 4e-6
+    y[:, :, 0, 0] = ref[:, :, 0, 0]
+    assert ((y - ref).norm() / (ref.square().sum() - ref[:, :, 0, 0].square().sum()).sqrt()).item() <= 4e-6
+
+
 # (shape, G, ATK_GN_CL_RESIDENT): which register-resident configuration the channels-last
 # forward takes ("0" = the three-kernel path).  With at least as many chunks per sample as
 # groups, one workgroup per group merges that group's chunk records (two-level); with fewer,
