@@ -913,8 +913,8 @@ int validate_gn(int64_t N, int64_t C, int64_t S, int G, int dtype, int variant) 
 //   dx = rstd * (g - mean_group(g) - x_hat * mean_group(g * x_hat)),
 //   dgamma_c = sum_{n,s} dy * x_hat,  dbeta_c = sum_{n,s} dy.
 // Two kernels, 5 tensor-passes of HBM traffic (x and dy read twice, dx written once):
-//   rows:     one workgroup per (n, c) row: x's mean / M2 about a row-wide shift K (the
-//             row's first element), A = sum dy, B = sum dy * (x - K);
+//   rows:     one workgroup per (n, c) row: x's mean / M2, A = sum dy, B = sum dy * (x - K), K a
+//             row-wide shift (the row's first element; for unaligned rows their mean);
 //   apply:    one workgroup per row: one wave merges the group's rows (Chan, fixed order, so
 //             every row of a group derives the same statistics), then dx.  The workgroups
 //             of n = 0 then also sum channel c's parameter gradients over n in a fixed
@@ -949,6 +949,18 @@ __device__ __forceinline__ void gn_st16u(void* p, uint4 r) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4_u*>(p));
 }
 
+// The median of three values of v (the first the mean of two, for 16-bit types all): a shift that one
+// far value among them does not move.
+template <typename T>
+__device__ __forceinline__ float vec_mid(const Vec16<T>& v) {
+  float t[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) t[k] = k < Vec16<T>::N ? to_f32(v.e[k]) : 0.f;
+  const float m = 0.5f * t[0] + 0.5f * t[1];
+  if constexpr (Vec16<T>::N == 4) return __builtin_amdgcn_fmed3f(m, t[2], t[3]);
+  else return __builtin_amdgcn_fmed3f(m, 0.5f * t[2] + 0.5f * t[3], 0.5f * t[4] + 0.5f * t[5]);
+}
+
 template <typename T, int U, bool RAG>
 __global__ __launch_bounds__(GN_TP_NT) void gn_bwd_rows_kernel(GnBwdArgs a) {
   constexpr int VEC = 16 / sizeof(T);
@@ -956,25 +968,21 @@ __global__ __launch_bounds__(GN_TP_NT) void gn_bwd_rows_kernel(GnBwdArgs a) {
   const int64_t r = blockIdx.x;
   const T* __restrict__ xr = static_cast<const T*>(a.x) + r * a.S;
   const T* __restrict__ gr = static_cast<const T*>(a.dy) + r * a.S;
-  // RAG: the mean of the row's first vector, nearer to the row's mean than one value, and each
-  // vector summed by itself first.  Both only for accuracy: fp32 dgamma over [3,448,33,54] against
-  // 64 bits 1.3e-7; with the one value and one running sum 1.8e-7
-  float K;
+  // RAG: each thread sums about a value of its own first vector, and the threads' moments are
+  // merged exactly: with one shift for the row, a value far from the rest in the row's first
+  // vector cancelled against the whole row (rstd off by 4e-5 with one of 1e3 in 20467).  Each
+  // vector is summed by itself first (fp32 dgamma over [3,448,33,54] against 64 bits 1.1e-7, with
+  // one running sum 1.8e-7).
+  float K = 0.f, K0 = 0.f;
   if constexpr (RAG) {
     Vec16<T> f;
     f.raw = gn_ld16u(xr);
-    float t[VEC];
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) t[k] = to_f32(f.e[k]) * (1.f / VEC);
-#pragma unroll
-    for (int h = VEC / 2; h; h >>= 1)
-#pragma unroll
-      for (int k = 0; k < h; ++k) t[k] += t[k + h];
-    K = t[0];
+    K0 = vec_mid(f);
   } else {
     K = to_f32(xr[0]);
   }
   float s1 = 0.f, s2 = 0.f, sa = 0.f, sb = 0.f;
+  int cnt = 0;  // RAG: the thread's elements
   // U vectors of x and of dy in flight per thread (branch-free buffer loads; vectors
   // past the row read zero and are masked out of the sums)
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(xr, (uint32_t)(a.S * (int64_t)sizeof(T)));
@@ -997,8 +1005,10 @@ __global__ __launch_bounds__(GN_TP_NT) void gn_bwd_rows_kernel(GnBwdArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if constexpr (RAG) {
+        if (u == 0 && e0 == (int64_t)threadIdx.x * VEC) K = vec_mid(xv[0]);
         const int64_t e = e0 + (int64_t)u * GN_TP_NT * VEC;
         const int skip = e >= a.S ? VEC : (int)max(e - (a.S - VEC), (int64_t)0);
+        cnt += VEC - skip;
         float d[VEC], g[VEC];
 #pragma unroll
         for (int k = 0; k < VEC; ++k) {
@@ -1030,6 +1040,17 @@ __global__ __launch_bounds__(GN_TP_NT) void gn_bwd_rows_kernel(GnBwdArgs a) {
         sb = fmaf(g, d, sb);
       }
     }
+  }
+  if constexpr (RAG) {
+    // the row's mean (about a value of its own, so that a common offset costs no precision), then
+    // this thread's M2 and B about it
+    const float n = (float)cnt, q = cnt ? s1 / n : 0.f, mt = K + q;
+    const float mean = K0 + block_sum<GN_TP_NT>(cnt ? n * (mt - K0) : 0.f, red) / (float)a.S;
+    const float d = cnt ? mt - mean : 0.f;
+    s2 = fmaf(n * d, d, fmaxf(fmaf(-s1, q, s2), 0.f));
+    sb = fmaf(K - mean, sa, sb);
+    s1 = 0.f;
+    K = mean;
   }
   // only thread 0 needs the totals: the four wave sums go through LDS in one exchange
   // (four block_sum calls would cost eight barriers in a workgroup this short-lived)

@@ -549,6 +549,23 @@ def test_group_norm_rows_of_any_length(dev, case, dtype):
         assert O.max_rel_err(db.cpu(), rdb) <= BWD_BAR_P[dtype]
 
 
+@pytest.mark.parametrize("far", [30.0, 1e3, 1e4])
+def test_group_norm_backward_any_length_far_value(dev, far):
+    """Unaligned rows whose first value is `far` times the spread from the rest.  A thread sums its
+    80 values of a row (20467) about one that the far value does not move, so nothing cancels:
+    M2 and the sums behind dgamma have the roundings of 20 vectors and of the merges, about 30 *
+    2^-24 = 2e-6 at worst, and rstd is the relative error of dx at the other positions."""
+    x, gm, _ = _inputs((2, 6, 211, 97), torch.float32, seed=11)
+    x[..., 0, 0] = far
+    dy = torch.randn(x.shape, generator=torch.Generator().manual_seed(12))
+    dx, dg, db = _native().group_norm_backward(dy.to(dev), x.to(dev), 3, gm.to(dev), 1e-5, (True, True, True))
+    rdx, rdg, rdb = (torch.as_tensor(t) for t in O.group_norm_bwd(x, 3, gm, dy, 1e-5))
+    d, rdx = dx.cpu().double() - rdx.view(x.shape), rdx.view(x.shape).clone()
+    d[..., 0, 0] = rdx[..., 0, 0] = 0
+    assert (d.norm() / rdx.norm()).item() <= 4e-6
+    assert O.max_rel_err(dg.cpu(), rdg) <= 4e-6 and O.max_rel_err(db.cpu(), rdb) <= 4e-6
+
+
 # Channel counts and groups off the column map of the channels-last kernels: groups of part of a
 # vector, groups that straddle vectors, vector counts that do not divide the workgroup, one group,
 # as many groups as threads, one position, chunks with a partial last row block
