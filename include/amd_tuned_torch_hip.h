@@ -262,6 +262,7 @@ int atk_dwconv1d_bwd(const void* x, const void* dy, const void* w, void* dx, flo
  * partial statistics and computed them itself -- results are exact either way).
  * The zeroed region has a fixed size and layout for every shape, so one workspace
  * serves calls of any shape (ordered on one stream), including HIP graph replays.
+ * The two-pass variant takes y == x; no other overlap of the two is allowed.
  * ------------------------------------------------------------------------- */
 size_t atk_group_norm_workspace_bytes(int64_t N, int64_t C, int64_t S, int G, int dtype,
                                       int variant);
@@ -334,7 +335,8 @@ int atk_group_norm_cl_fwd(const void* x, const void* gamma, const void* beta, vo
  * x, dy, dx: [N, C, S] of `dtype`; gamma: [C] of `param_dtype` or NULL (ones);
  * dgamma / dbeta: [C] fp32.  Any of dx / dgamma / dbeta may be NULL.  The group
  * statistics are recomputed from x with the forward's eps.  Needs S * sizeof(dtype)
- * of at least 16 (else ATK_UNSUPPORTED); rows of any length and element alignment.
+ * of at least 16 (else ATK_UNSUPPORTED); rows of any length and element alignment, those that
+ * are not 16-byte aligned with a dx apart from x and dy (else ATK_UNSUPPORTED).
  * The first 16 KiB of the workspace (atk_group_norm_bwd_workspace_bytes) must be zero
  * before the first call that uses it; every call leaves them zero (per-group counters).
  * Sums over n are taken in a fixed order (deterministic).  Groups of up to 8192 16-byte

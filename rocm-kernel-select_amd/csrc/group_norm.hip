@@ -3402,6 +3402,9 @@ extern "C" int atk_group_norm_bwd(const void* x, const void* dy, const void* gam
   // rows that are no multiple of 16 bytes, or misaligned tensors, take the rows / apply pair with
   // vectors at any address ([8, 256, 45, 45] bf16: 5.9 + 8.2 us against about 190 us in torch ops)
   const bool ragged = S % vec || !aligned16(x) || !aligned16(dy) || (dx && !aligned16(dx));
+  // (a row's last vector is read again by the thread before it after that one's may have been stored)
+  if (ragged && dx && (dx == x || dx == dy))
+    return fail(ATK_UNSUPPORTED, "group_norm backward: unaligned rows cannot be overwritten in place");
   if (S < vec) return fail(ATK_UNSUPPORTED, "group_norm backward: needs a spatial size of at least %lld", (long long)vec);
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(dx)) & (uintptr_t)(es - 1))
     return fail(ATK_EINVAL, "group_norm backward: misaligned element pointer");

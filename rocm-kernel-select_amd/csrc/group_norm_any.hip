@@ -25,7 +25,8 @@ __device__ __forceinline__ void st16u_nt(void* p, uint4 r) {
 // NC[S] rows of any length.  A group is E = cpg * S consecutive elements, read as 16-byte vectors
 // from its first element on, whatever its address; the last vector, where E is no multiple of
 // one, is read as the group's last 16 bytes.  Elements that it shares with the vector before are
-// left out of the sums and stored twice with the same value.
+// left out of the sums, and stored twice with the same value where the group is held in
+// registers, once where it is read again.  y may be x.
 // ---------------------------------------------------------------------------------------
 constexpr int GA_AFF = 1024;  // channels per group whose scale and shift fit LDS
 constexpr int GA_NT = 256;    // threads of the two-pass kernels
@@ -189,8 +190,8 @@ __global__ __launch_bounds__(GA_NT) void gn_any_apply_kernel(GaArgs a) {
   const int tid = threadIdx.x;
   const int64_t gi = blockIdx.x / a.NS, s = blockIdx.x - gi * a.NS;
   const int64_t s0 = s * a.slice, s1 = min(s0 + a.slice, a.E);
-  const T* __restrict__ xg = static_cast<const T*>(a.x) + gi * a.E;
-  T* __restrict__ yg = static_cast<T*>(a.y) + gi * a.E;
+  const T* xg = static_cast<const T*>(a.x) + gi * a.E;
+  T* yg = static_cast<T*>(a.y) + gi * a.E;
   Vec16<T> v[U];
   auto issue = [&](int64_t e0) {
 #pragma unroll
@@ -222,10 +223,19 @@ __global__ __launch_bounds__(GA_NT) void gn_any_apply_kernel(GaArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t e = e0 + (int64_t)u * GA_NT * VEC, em = min(e, a.E - VEC);
-      if (e < s1)
-        st16u_nt(yg + em, apply_vec<T, SILU>(v[u], (uint32_t)em, a, [&](uint32_t c, float& sc, float& sh) {
-                   affine_of(a, c0 + c, mean, rstd, sc, sh);
-                 }));
+      if (e >= s1) continue;
+      Vec16<T> o;
+      o.raw = apply_vec<T, SILU>(v[u], (uint32_t)em, a, [&](uint32_t c, float& sc, float& sh) {
+        affine_of(a, c0 + c, mean, rstd, sc, sh);
+      });
+      if (em == e) {
+        st16u_nt(yg + e, o.raw);
+      } else {  // the elements shared with the vector before belong to its thread: y may be x, normalised there already
+        const int own = (int)(e - em);
+#pragma unroll
+        for (int k = 1; k < VEC; ++k)
+          if (k >= own) yg[em + k] = o.e[k];
+      }
     }
   }
 }

@@ -141,6 +141,17 @@ def test_argument_validation_codes(nat):
     assert "alias" in nat.last_error()
 
 
+def test_group_norm_backward_refuses_unaligned_rows_in_place(nat):
+    """A row's last vector overlaps the one before it and is read after that may be stored, so dx
+    may be neither x nor dy there.  Host checks only: the pointers are never read."""
+    lib = nat.lib()
+    x, dy, ws, ws_bytes = 1 << 20, 2 << 20, 3 << 20, lib.atk_group_norm_bwd_workspace_bytes(2, 4)
+    for dx in (x, dy):
+        assert lib.atk_group_norm_bwd(x, dy, None, dx, None, None, 2, 4, 7, 2, 1e-5, 0, 0, ws, ws_bytes,
+                                      None) == nat.ATK_UNSUPPORTED
+        assert "in place" in nat.last_error()
+
+
 def _fastdiv(n, d):
     """Round-up multiplier method as atk_common.h implements it (32-bit)."""
     s = 0

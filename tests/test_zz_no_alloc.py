@@ -52,6 +52,22 @@ def test_group_norm_noalloc_matches_workspace_entry_point(dev, name):
     assert not nat.group_norm_barrier_error(dev)
 
 
+@pytest.mark.parametrize("shape,G", [((2, 12, 211, 97), 3), ((1, 4, 257, 255), 1), ((2, 16, 45, 45), 4),
+                                     ((1, 32, 64, 64), 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_group_norm_in_place(dev, shape, G, dtype):
+    """The two-pass variant with y == x, on unaligned rows (whose last vector overlaps the one before)
+    and aligned ones, gives the bits of a separate output."""
+    nat = _native()
+    x, gm, bt = _inputs(shape, dtype, 6)
+    xd, gd, bd = x.to(dev), gm.to(dev), bt.to(dev)
+    vi = nat.variants(nat.OP_GROUP_NORM).index("twopass")
+    want = nat.group_norm(xd, G, gd, bd, 1e-5, variant=vi)
+    buf = xd.clone()
+    assert nat.group_norm_noalloc(buf, G, buf, gd, bd, 1e-5, variant=vi) is buf
+    assert torch.equal(buf, want)
+
+
 def test_group_norm_noalloc_rejects_shapes_beyond_the_scratch(dev):
     """Two-pass partials above the static scratch's 1 MiB (262144 groups here) are refused
     with a clear error; nothing is launched."""
