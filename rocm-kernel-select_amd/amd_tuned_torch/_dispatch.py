@@ -409,7 +409,8 @@ def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups,
     """(dw, db) through the native kernel for stride-1, dilation-1, groups-1 'same' convs with
     3x3 (2D) or 3x3x3 / 1x3x3 (3D) kernels in 16-bit types, db (the sum of dy, in the weight's
     dtype) only with `bias_grad`; None otherwise (or when the kernel declines the shape)."""
-    if groups != 1 or isinstance(padding, str) or weight.dtype not in (torch.float16, torch.bfloat16):
+    if (groups != 1 or isinstance(padding, str) or weight.dtype not in (torch.float16, torch.bfloat16)
+            or not _native.available()):
         return None
     tup = _triple if nd == 3 else _pair
     try:

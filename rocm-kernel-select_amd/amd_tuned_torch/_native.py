@@ -1449,13 +1449,16 @@ def group_norm_apply(x: torch.Tensor, num_groups: int, weight: Optional[torch.Te
 def conv_dgrad_weight(weight: torch.Tensor) -> torch.Tensor:
     """weight [Co, Ci, *k] -> [Ci, Co, *k] with every spatial axis flipped, contiguous: the weights
     of the forward conv that computes the input gradient of a stride-1 conv."""
-    if not (weight.is_cuda and weight.is_contiguous() and weight.dtype in _DTYPE_CODE and weight.numel()):
-        return weight.transpose(0, 1).flip(list(range(2, weight.dim()))).contiguous()
-    Co, Ci = weight.shape[:2]
-    wt = torch.empty((Ci, Co) + tuple(weight.shape[2:]), dtype=weight.dtype, device=weight.device)
-    _check(lib().atk_conv_dgrad_weight(weight.data_ptr(), wt.data_ptr(), Co, Ci, weight.numel() // (Co * Ci),
-                                       _DTYPE_CODE[weight.dtype], _stream(weight)), "conv_dgrad_weight")
-    return wt
+    if weight.is_cuda and weight.is_contiguous() and weight.dtype in _DTYPE_CODE and weight.numel() and available():
+        Co, Ci = weight.shape[:2]
+        wt = torch.empty((Ci, Co) + tuple(weight.shape[2:]), dtype=weight.dtype, device=weight.device)
+        try:
+            _check(lib().atk_conv_dgrad_weight(weight.data_ptr(), wt.data_ptr(), Co, Ci, weight.numel() // (Co * Ci),
+                                               _DTYPE_CODE[weight.dtype], _stream(weight)), "conv_dgrad_weight")
+            return wt
+        except Unsupported:  # 2^30 weights and more
+            pass
+    return weight.transpose(0, 1).flip(list(range(2, weight.dim()))).contiguous()
 
 
 def conv_wgrad(x: torch.Tensor, dy: torch.Tensor, kd: int, *, bias_grad: bool = False,

@@ -424,6 +424,47 @@ def test_conv_autograd_wrapper_backward(monkeypatch):
         torch.testing.assert_close(a, r)
 
 
+class _Gpu(torch.Tensor):
+    """A CPU tensor that says it is on the GPU (the native layer is out of reach in these tests)."""
+    is_cuda = property(lambda self: True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_conv_backward_without_the_library(monkeypatch, dtype):
+    """With no loadable library the patched forward is stock's, and so must the backward be: no
+    gradient may ask for the library."""
+    def no_lib():
+        raise AssertionError("the library was asked for")
+    monkeypatch.setattr(_native, "available", lambda: False)
+    monkeypatch.setattr(_native, "lib", no_lib)
+    g = torch.Generator().manual_seed(3)
+    x, dy = torch.randn(2, 4, 9, 10, generator=g).to(dtype), torch.randn(2, 6, 9, 10, generator=g).to(dtype)
+    w = torch.randn(6, 4, 3, 3, generator=g).to(dtype)
+    orig = _dispatch._ORIGINALS[(F, "conv2d")]
+    got = _dispatch._conv_grads(*(t.as_subclass(_Gpu) for t in (dy, x, w)), [6], (1, 1, 1, 1, 2),
+                                [True, True, True], lambda *a: orig(*a))
+    ref = torch.ops.aten.convolution_backward(dy.double(), x.double(), w.double(), [6], [1, 1], [1, 1], [1, 1], False,
+                                              [0, 0], 1, [True, True, True])
+    bar = 1e-5 if dtype == torch.float32 else 1e-2
+    for a, r in zip(got, ref):
+        assert (a.as_subclass(torch.Tensor).double() - r).abs().max() <= bar * r.abs().max()
+
+
+def test_conv_dgrad_weight_declined_by_the_library(monkeypatch):
+    """Too many weights for the kernel: the torch form."""
+    class Lib:
+        @staticmethod
+        def atk_conv_dgrad_weight(*a):
+            return _native.ATK_UNSUPPORTED
+    monkeypatch.setattr(_native, "available", lambda: True)
+    monkeypatch.setattr(_native, "lib", lambda: Lib)
+    monkeypatch.setattr(_native, "last_error", lambda: "too many weights")
+    monkeypatch.setattr(_native, "_stream", lambda t: 0)
+    w = torch.randn(3, 2, 3, 4)
+    got = _native.conv_dgrad_weight(w.as_subclass(_Gpu))
+    assert torch.equal(got.as_subclass(torch.Tensor), w.transpose(0, 1).flip([2, 3]))
+
+
 def test_dwconv1d_autograd_backward_matches_stock(monkeypatch):
     """The depthwise conv1d autograd wrapper's backward (stock convolution_backward on the
     left/right padded input) equals autograd through stock F.conv1d, for the symmetric,
