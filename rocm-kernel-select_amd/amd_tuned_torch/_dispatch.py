@@ -24,6 +24,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _native
+from . import autograd_state
 from . import compile_ops
 from . import conv_fusion_ops
 from . import kernel_select
@@ -439,24 +440,18 @@ def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups,
     return dw.view(weight.shape).to(weight.dtype), None if db is None else db.to(weight.dtype)
 
 
-def _graph_wanted(*tensors) -> bool:
-    """True when the gradients being computed are to be differentiated again (create_graph=True):
-    the native backward kernels record nothing, so they must not serve the call."""
-    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
-
-
 def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
     """(dx, dw, db) of a patched conv for `needs` = [dx, dw, db] wanted:
     * dx of a stride-1, dilation-1, groups-1 conv through `fwd` (the accelerated forward) on dy
       with transposed, flipped weights;
     * dw of a 'same' 3x3(x3) conv in a 16-bit type through the native wgrad kernel, db with it;
     * db alone as a reduction of dy once every other gradient is native;
-    * whatever is left, and everything that is to be differentiated again, through
+    * whatever is left, and everything that must be differentiable itself (graph_wanted), through
       aten.convolution_backward, the op autograd uses unpatched."""
     stride, padding, dilation, groups, nd = conf
     needs = list(needs)
     gi = gw = gb = None
-    native = input.is_cuda and not _graph_wanted(grad_output, input, weight)
+    native = input.is_cuda and not autograd_state.graph_wanted(grad_output, input, weight)
     if needs[0] and native:
         pad_t = _dgrad_padding(weight, stride, padding, dilation, groups, nd)
         if pad_t is not None:
@@ -554,6 +549,8 @@ def _patched_conv2d(input, weight, bias=None, stride=1, padding=0, dilation=1, g
                 and _is_pointwise_conv2d(weight, stride, padding, dilation)):
             return orig(input, weight, bias, stride, padding, dilation, groups)
         return _traced_conv(2, input, weight, bias, stride, padding, dilation, groups, orig)
+    if autograd_state.transformed(input, weight, bias):
+        return orig(input, weight, bias, stride, padding, dilation, groups)
     if groups != 1:
         if _DEBUG:
             _debug("conv2d", "stock", "grouped conv: no tier here supports groups != 1",
@@ -580,6 +577,8 @@ def _patched_conv3d(input, weight, bias=None, stride=1, padding=0, dilation=1, g
     orig = _STOCK_F["conv3d"]
     if _is_compiling():
         return _traced_conv(3, input, weight, bias, stride, padding, dilation, groups, orig)
+    if autograd_state.transformed(input, weight, bias):
+        return orig(input, weight, bias, stride, padding, dilation, groups)
 
     def fwd(i, w, b, s, p, d, g):
         return _conv_accelerated_forward(3, i, w, b, s, p, d, g, orig)
@@ -747,11 +746,11 @@ def _group_norm_grads(grad_output, input, num_groups, weight, eps, needs):
     backward kernels for contiguous or channels-last GPU input (channels-last first on the
     channels-last kernels, else through NC[S] copies made by the native transpose, dx coming
     back in the input's layout; dgamma / dbeta in fp32), the textbook torch-op backward
-    otherwise (dgamma / dbeta in the parameter dtypes).  Gradients that are to be differentiated
-    again take the torch ops too, 16-bit ones on the GPU in fp32, as the kernels compute.
+    otherwise (dgamma / dbeta in the parameter dtypes).  Gradients that must be differentiable
+    themselves (graph_wanted) take the torch ops too, 16-bit ones on the GPU in fp32, as the kernels compute.
     Entries not asked for are None."""
     cl = _channels_last(input)
-    if input.is_cuda and _graph_wanted(grad_output, input, weight):
+    if input.is_cuda and autograd_state.graph_wanted(grad_output, input, weight):
         acc = torch.promote_types(input.dtype, torch.float32)
         gx, gw, gb = _group_norm_backward(grad_output.to(acc).contiguous(), input.to(acc), num_groups,
                                           None if weight is None else weight.to(acc), eps, needs)
@@ -817,6 +816,8 @@ def _traced_group_norm(input, num_groups, weight, bias, eps, orig):
 def _patched_group_norm(input, num_groups, weight=None, bias=None, eps=1e-5):
     if _is_compiling():
         return _traced_group_norm(input, num_groups, weight, bias, eps, _STOCK_F["group_norm"])
+    if autograd_state.transformed(input, weight, bias):
+        return _STOCK_F["group_norm"](input, num_groups, weight, bias, eps)
     if _grad_safe(input, weight, bias):
         return _group_norm_accelerated_forward(input, num_groups, weight, bias, eps)
     if _DEBUG:

@@ -19,6 +19,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _native
+from . import autograd_state
 from . import compile_ops
 from . import kernel_select
 
@@ -52,7 +53,8 @@ def _layout(x: torch.Tensor) -> str:
 
 def _eligible(x, num_groups, weight, bias, layout_ok: bool = False) -> bool:
     """Native-eligible input: enabled, GPU, a supported dtype, contiguous (or, with
-    layout_ok, any layout the caller handles), plain tensor types, no gradient needed."""
+    layout_ok, any layout the caller handles), plain tensor types, no gradient needed, no
+    tangent or transform to carry."""
     if not (enabled() and isinstance(x, torch.Tensor) and x.is_cuda and x.dim() >= 3
             and x.dtype in _DTYPES and (layout_ok or x.is_contiguous())
             and type(x) in (torch.Tensor, nn.Parameter)):
@@ -65,7 +67,7 @@ def _eligible(x, num_groups, weight, bias, layout_ok: bool = False) -> bool:
     if torch.is_grad_enabled() and (x.requires_grad or (weight is not None and weight.requires_grad)
                                     or (bias is not None and bias.requires_grad)):
         return False
-    return True
+    return not autograd_state.transformed(x, weight, bias)
 
 
 def _grad_needed(x, weight, bias) -> bool:
@@ -211,7 +213,7 @@ def conv_residual(input: torch.Tensor, weight: torch.Tensor, bias: Optional[torc
         return stock_conv(input, weight, bias, stride, padding, dilation) + residual
 
     if (nd not in (2, 3) or _grad_needed(input, weight, bias) or _grad_needed(residual, None, None)
-            or compile_ops.is_compiling()
+            or compile_ops.is_compiling() or autograd_state.transformed(input, weight, bias, residual)
             or not _conv_geometry_ok(input, weight, bias, residual, stride, padding, dilation)):
         return (stock_conv(input, weight, bias, stride, padding, dilation) if stock_conv is not None
                 else F.conv3d(input, weight, bias, stride, padding, dilation)) + residual
@@ -267,7 +269,8 @@ def conv_group_norm_silu(input: torch.Tensor, weight: torch.Tensor, bias: Option
                                                                                           beta, eps)
 
     if (nd not in (2, 3) or compile_ops.is_compiling() or _grad_needed(input, weight, bias)
-            or _grad_needed(gamma, beta, None) or not enabled()
+            or _grad_needed(gamma, beta, None) or autograd_state.transformed(input, weight, bias, gamma, beta)
+            or not enabled()
             or not _conv_geometry_ok(input, weight, bias, None, stride, padding, dilation)
             or not isinstance(num_groups, int) or num_groups <= 0 or weight.shape[0] % num_groups
             or any(p is not None and (not p.is_cuda or p.dtype not in _DTYPES) for p in (gamma, beta))):

@@ -28,6 +28,7 @@ from typing import Any, Callable, Optional
 import torch
 
 from . import _native
+from . import autograd_state
 from . import compile_ops
 from . import depthwise_conv1d_ops
 from . import kernel_select
@@ -347,6 +348,8 @@ def _miopen_safe_conv(op_name: str, orig_fn: Callable) -> Callable:
         if compile_ops.is_compiling():
             return _traced_conv1d(input, weight, bias, stride, padding, dilation, groups, orig_fn)
         args = (input, weight, bias, stride, padding, dilation, groups)
+        if autograd_state.transformed(input, weight, bias):
+            return _stock_with_rescue(op_name, orig_fn, *args)
         for fast_path in (_try_causal_conv1d_fastpath, _try_channel_last_fastpath):
             out = fast_path(*args)
             if out is not None:

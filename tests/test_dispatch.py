@@ -14,6 +14,7 @@ import amd_tuned_torch as att
 from amd_tuned_torch import _dispatch, _native, conv_fusion_ops, kernel_select, miopen_fallback
 
 STOCK_CONV1D = miopen_fallback._original_conv1d
+STOCK_GROUP_NORM = _dispatch._STOCK_F["group_norm"]
 
 
 # ---------------------------------------------------------------------------
@@ -270,6 +271,83 @@ def test_group_norm_contest_and_key(monkeypatch, contest):
     fake.calls.clear()
     F.group_norm(x.transpose(2, 3), 4)
     assert fake.calls == []
+
+
+def test_tangents_and_transforms_take_stock(monkeypatch):
+    """A native kernel would drop a forward-mode tangent and cannot read a functorch wrapper: dual
+    tensors, jvp, vmap and grad run stock; a forward-mode level alone changes nothing."""
+    import torch.autograd.forward_ad as fwad
+    monkeypatch.setattr(kernel_select, "_ENABLED", False)
+    fake = FakeNative(monkeypatch, ["f32_a"], ["twopass"])
+
+    def cl(x, G, w=None, b=None, eps=1e-5, *, silu=False, out=None):
+        fake.calls.append(("group_norm_cl", "cl"))
+        return STOCK_GROUP_NORM(x.detach(), G, w, b, eps)
+    monkeypatch.setattr(_native, "group_norm_cl", cl)
+    g = torch.Generator().manual_seed(4)
+    x, t = torch.randn(2, 8, 5, 6, generator=g), torch.randn(2, 8, 5, 6, generator=g)
+    wc, wn = torch.randn(4, 8, 3, 3, generator=g), torch.randn(8, generator=g)
+    last = dict(memory_format=torch.channels_last)
+
+    def dual(f, x, t):
+        with fwad.dual_level():
+            y = fwad.unpack_dual(f(fwad.make_dual(x, t)))
+            assert y.tangent is not None
+            return tuple(y)
+
+    def outcome(run, f):  # (stock has no tangent of a channels-last GroupNorm: it raises)
+        try:
+            return run(f)
+        except RuntimeError as e:
+            return str(e)
+
+    cases = [(lambda v: F.group_norm(v, 4, wn), lambda v: STOCK_GROUP_NORM(v, 4, wn), x, t),
+             (lambda v: F.group_norm(v, 4, wn), lambda v: STOCK_GROUP_NORM(v, 4, wn), x.contiguous(**last),
+              t.contiguous(**last)),
+             (lambda v: F.conv2d(v, wc, None, 1, 1), lambda v: torch.conv2d(v, wc, None, 1, 1), x, t)]
+    for fn, stock, x, t in cases:
+        fn(x)
+        with fwad.dual_level():
+            fn(x)
+            assert len(fake.calls) == 2, "plain tensors, with and without a level, run native"
+        xs = torch.stack([x, t])
+        for run in (lambda f: dual(f, x, t), lambda f: torch.func.jvp(f, (x,), (t,)), lambda f: torch.func.vmap(f)(xs),
+                    lambda f: torch.func.grad(lambda v: f(v).square().sum())(x)):
+            a, b = outcome(run, fn), outcome(run, stock)
+            assert a == b if isinstance(b, str) else torch.testing.assert_close(a, b) is None
+        assert len(fake.calls) == 2
+        fake.calls.clear()
+
+
+def test_dual_and_batched_gradients_take_differentiable_ops(monkeypatch):
+    """In a backward whose incoming gradient is batched or carries a tangent no native kernel runs
+    (the input says that it is on the GPU)."""
+    import torch.autograd.forward_ad as fwad
+
+    def native(*a, **k):
+        raise AssertionError("a native kernel was asked for")
+    for name in ("conv_wgrad", "conv_dgrad_weight", "group_norm_backward", "group_norm_cl_backward"):
+        monkeypatch.setattr(_native, name, native)
+    monkeypatch.setattr(_native, "available", lambda: True)
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(2, 8, 5, 9, generator=g)
+    w, gm = torch.randn(4, 8, 3, 3, generator=g), torch.randn(8, generator=g)
+    ops = [(_dispatch._ConvFn, (w, torch.zeros(4), 1, 1, 1, 1, 2, lambda *a: torch.conv2d(*a)),
+            lambda v: torch.conv2d(v, w, torch.zeros(4), 1, 1)),
+           (_dispatch._GroupNormFn, (gm, None, 4, 1e-5), lambda v: STOCK_GROUP_NORM(v, 4, gm, None, 1e-5))]
+    monkeypatch.setattr(_dispatch, "_group_norm_accelerated_forward", STOCK_GROUP_NORM)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    for fn, args, stock in ops:
+        v = x.clone().requires_grad_()
+        y, ref = fn.apply(v, *args), stock(v)
+        dy, t = torch.randn(y.shape, generator=g), torch.randn(y.shape, generator=g)
+        both = torch.stack([dy, t])
+        for a, r in zip(torch.autograd.grad(y, v, both, is_grads_batched=True, retain_graph=True),
+                        torch.autograd.grad(ref, v, both, is_grads_batched=True, retain_graph=True)):
+            torch.testing.assert_close(a, r)
+        with fwad.dual_level():
+            a = fwad.unpack_dual(torch.autograd.grad(y, v, fwad.make_dual(dy, t), retain_graph=True)[0])
+        torch.testing.assert_close(a.tangent, torch.autograd.grad(ref, v, t)[0])  # dx is linear in dy
 
 
 def test_kernel_select_off_uses_fixed_native_order(monkeypatch):
