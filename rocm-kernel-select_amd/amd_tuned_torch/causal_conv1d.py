@@ -27,6 +27,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _native
+from . import autograd_state
 
 
 def _channel_last(x: torch.Tensor) -> bool:
@@ -117,6 +118,34 @@ def _backward(x, weight, bias, dout, seq_idx, initial_states, dfinal, silu: bool
     return dx, dw.to(weight.dtype), (db.to(bias.dtype) if bias is not None else None), dinit
 
 
+def _backward_ops(x, weight, bias, dout, seq_idx, initial_states, dfinal, silu: bool):
+    """_backward in differentiable torch ops, fp32, for gradients that are to be differentiated
+    again or whose incoming gradient is batched or dual (the kernels record nothing)."""
+    L, H = x.shape[2], weight.shape[1] - 1
+    acc = torch.promote_types(x.dtype, torch.float32)
+    w, b = _kernel_weight(weight, x, bias)
+    w = w.to(acc)
+    context = x.new_zeros(x.shape[:2] + (H,)) if initial_states is None else initial_states
+    xp = torch.cat([context.to(acc), x.to(acc)], dim=-1)
+    seq = None if seq_idx is None else F.pad(seq_idx, (H, 0), value=-1).unsqueeze(1)
+
+    def own(v, j):  # v where tap j stays in its output's sequence, zero elsewhere
+        return v if seq is None else torch.where(seq[..., j:j + L] == seq[..., H:], v, torch.zeros_like(v))
+
+    taps = [own(xp[..., j:j + L], j) for j in range(H + 1)]
+    g = dout.to(acc)
+    if silu:
+        z = sum(w[:, j, None] * t for j, t in enumerate(taps))
+        g = g * _dsilu(z if b is None else z + b.to(acc)[:, None])
+    dxp = sum(F.pad(own(g * w[:, j, None], j), (j, H - j)) for j in range(H + 1))
+    if dfinal is not None:
+        dxp = dxp + F.pad(dfinal.to(acc), (L, 0))
+    dw = torch.stack([(g * t).sum(dim=(0, 2)) for t in taps], dim=-1)
+    return (dxp[..., H:].to(x.dtype), dw.to(weight.dtype),
+            None if bias is None else g.sum(dim=(0, 2)).to(bias.dtype),
+            None if initial_states is None else dxp[..., :H].to(initial_states.dtype))
+
+
 def _checked(x, weight, bias, activation):
     """(x, bias) as the kernels take them, after the interface's argument checks."""
     if activation not in (None, "silu", "swish"):
@@ -184,6 +213,10 @@ class CausalConv1dFn(torch.autograd.Function):
     def backward(ctx, dout, *args):
         x, weight, bias, seq_idx, initial_states = ctx.saved_tensors
         dfinal = args[0] if ctx.return_final_states else None
+        if autograd_state.graph_wanted(dout, x, weight, bias, initial_states, dfinal):
+            dx, dweight, dbias, dinit = _backward_ops(x, weight, bias, dout, seq_idx, initial_states, dfinal,
+                                                      ctx.activation)
+            return dx, dweight, dbias, None, dinit, None, None, None
         if dout.stride(2) != 1 and dout.stride(1) != 1:
             dout = dout.contiguous()
         dx, dweight, dbias, dinit = _backward(x, weight, bias, dout, seq_idx, initial_states, dfinal,

@@ -19,6 +19,8 @@ from typing import Any, Optional, Tuple
 import torch
 
 from . import _native
+from . import autograd_state
+from . import compile_ops
 
 KMAX = 64
 PADMAX = 64
@@ -201,6 +203,11 @@ class DepthwiseConv1dFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         input, weight, bias = ctx.saved_tensors
+        if not compile_ops.is_compiling() and autograd_state.graph_wanted(dout, input, weight):
+            # differentiable themselves, in the wider of the types (fp32 weights enter unrounded)
+            acc = torch.promote_types(input.dtype, weight.dtype)
+            du, dw, db = _stock_backward(dout.to(acc), input.to(acc), weight.to(acc), bias, ctx.padding, ctx.is_bhl)
+            return du.to(input.dtype), dw.to(weight.dtype), db.to(bias.dtype), None, None
         du, dw, db = conv1d_backward(dout, input, weight, bias, ctx.padding, ctx.is_bhl)
         return du, dw, db, None, None
 

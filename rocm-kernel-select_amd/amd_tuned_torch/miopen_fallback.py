@@ -130,7 +130,7 @@ class _DwConv1dFn(torch.autograd.Function):
     """Native forward; native backward where the library serves it (input gradient through
     the forward kernel with reversed weights when pad_left <= K-1, weight and bias gradients
     through the streaming reduction kernel when K <= 5), stock aten.convolution_backward for
-    the rest."""
+    the rest and for gradients that must be differentiable themselves."""
 
     @staticmethod
     def forward(ctx, input, weight, bias, pad_left, l_out, variant):
@@ -147,7 +147,7 @@ class _DwConv1dFn(torch.autograd.Function):
         needs = [bool(ctx.needs_input_grad[0]), bool(ctx.needs_input_grad[1]),
                  ctx.has_bias and bool(ctx.needs_input_grad[2])]
         gi = gw = gb = None
-        if dout.is_cuda and _native.available():
+        if dout.is_cuda and _native.available() and not autograd_state.graph_wanted(dout, input, weight):
             dout = dout.contiguous()
             x = input.detach()
             if needs[0]:
@@ -182,7 +182,7 @@ class _DwConv1dFn(torch.autograd.Function):
         L = input.shape[-1]
         # stock semantics of a left-pad / right-crop: pad so the stock conv spans l_out
         pad_right = ctx.l_out - (L + ctx.pad_left - K + 1)
-        xin = torch.nn.functional.pad(input.detach(), (ctx.pad_left, max(0, pad_right)))
+        xin = torch.nn.functional.pad(input, (ctx.pad_left, max(0, pad_right)))
         if pad_right < 0:
             xin = xin[..., :xin.shape[-1] + pad_right]
         gi, gw, gb = torch.ops.aten.convolution_backward(

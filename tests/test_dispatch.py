@@ -565,6 +565,82 @@ def test_dwconv1d_autograd_backward_matches_stock(monkeypatch):
             torch.testing.assert_close(a, r)
 
 
+def test_conv1d_functions_second_derivatives(monkeypatch):
+    """Gradients taken with create_graph=True through the depthwise and causal conv1d functions
+    carry the graph of every input (float64, against autograd through the plain formulas)."""
+    from amd_tuned_torch import causal_conv1d as cc, depthwise_conv1d_ops as dwo
+    g = torch.Generator().manual_seed(8)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, dtype=torch.float64)
+
+    def fake_dw(x, w, b, pad_left, l_out, silu=False, variant=-1, out=None):
+        w = w.reshape(x.shape[1], 1, -1)
+        xp = F.pad(x, (pad_left, max(0, l_out + w.shape[2] - 1 - x.shape[-1] - pad_left)))
+        y = STOCK_CONV1D(xp, w, b, 1, 0, 1, x.shape[1])[..., :l_out]
+        return F.silu(y) if silu else y
+
+    def fake_cl(x, w, b, pad, l_out, *, silu, seq_idx, seq_mode, initial_states, final_states, out):
+        y, fin = states(x.transpose(1, 2), w, b, seq_idx, None if initial_states is None
+                        else initial_states.transpose(1, 2), silu)
+        out.copy_(y.transpose(1, 2))
+        if final_states is not None:
+            final_states.copy_(fin.transpose(1, 2))
+
+    def states(x, w, b, seq_idx, init, silu=True):
+        H, L = w.shape[1] - 1, x.shape[2]
+        xp = torch.cat([x.new_zeros(x.shape[:2] + (H,)) if init is None else init, x], dim=-1)
+        z = b[:, None]
+        for j in range(H + 1):
+            tap = xp[..., j:j + L]
+            if seq_idx is not None:
+                at = [t - H + j for t in range(L)]
+                m = torch.stack([(seq_idx[:, p] == seq_idx[:, t]) if p >= 0 else torch.zeros(len(x), dtype=torch.bool)
+                                 for t, p in enumerate(at)], dim=1)
+                tap = torch.where(m[:, None], tap, torch.zeros_like(tap))
+            z = z + w[:, j, None] * tap
+        return F.silu(z) if silu else z, xp[..., L:]
+
+    monkeypatch.setattr(_native, "dwconv1d", fake_dw)
+    monkeypatch.setattr(_native, "dwconv1d_cl", fake_cl)
+    monkeypatch.setattr(dwo, "_fwd_impl", lambda x, w, b, p, bhl: fake_dw(x, w, b, p, x.shape[2] + 2 * p - w.shape[1] + 1)
+                        if bhl else fake_dw(x.transpose(1, 2), w.t(), b, p, x.shape[1] + 2 * p - w.shape[0] + 1)
+                        .transpose(1, 2))
+    x, w, b, init = rand(2, 3, 7), rand(3, 4), rand(3), rand(2, 3, 3)
+    seq = torch.tensor([[0, 0, 0, 1, 1, 2, 2], [5, 5, 6, 6, 6, 6, 6]], dtype=torch.int32)
+
+    def last(t):  # (B, D, L) with unit channel stride
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+    cases = [
+        (lambda x, w, b: miopen_fallback._DwConv1dFn.apply(x, w.unsqueeze(1), b, 3, 10, -1),
+         lambda x, w, b: STOCK_CONV1D(x, w.unsqueeze(1), b, 1, 3, 1, 3), (x, w, b)),
+        (lambda x, w, b: dwo.DepthwiseConv1dFn.apply(x, w, b, 2, True),
+         lambda x, w, b: STOCK_CONV1D(x, w.unsqueeze(1), b, 1, 2, 1, 3), (x, w, b)),
+        (lambda x, w, b: dwo.DepthwiseConv1dFn.apply(x.transpose(1, 2), w.t(), b, 2, False).transpose(1, 2),
+         lambda x, w, b: STOCK_CONV1D(x, w.unsqueeze(1), b, 1, 2, 1, 3), (x, w, b)),
+        (lambda x, w, b: cc.causal_conv1d_fn(x, w, b, activation="silu"),
+         lambda x, w, b: states(x, w, b, None, None)[0], (x, w, b)),
+        (lambda x, w, b: cc.causal_conv1d_fn(last(x), w, b, seq_idx=seq, activation="silu"),
+         lambda x, w, b: states(x, w, b, seq, None)[0], (x, w, b)),
+        (lambda x, w, b, i: torch.cat(cc.causal_conv1d_fn(last(x), w, b, initial_states=last(i),
+                                                          return_final_states=True, activation="silu"), dim=-1),
+         lambda x, w, b, i: torch.cat(states(x, w, b, None, i), dim=-1), (x, w, b, init)),
+    ]
+    for fn, plain, args in cases:
+        v = [rand(*t.shape) for t in args]
+        dy = rand(*plain(*args).shape)
+        results = []
+        for f in (fn, plain):
+            leaves = [t.clone().requires_grad_() for t in args]
+            up = dy.clone().requires_grad_()
+            first = torch.autograd.grad(f(*leaves), leaves, up, create_graph=True)
+            total = sum((a * c).sum() for a, c in zip(first, v))
+            results.append(first + torch.autograd.grad(total, [up] + leaves, allow_unused=True, materialize_grads=True))
+        for a, r in zip(*results):
+            torch.testing.assert_close(a, r, rtol=1e-6, atol=1e-6)
+
+
 def test_conv1d_padding_resolution():
     assert miopen_fallback._resolve_padding(1, 3, 10) == (1, 10)
     assert miopen_fallback._resolve_padding((3,), 4, 10) == (3, 13)

@@ -47,6 +47,24 @@ def test_conv2d(ci, co, size):
              (2, co) + size, torch.float16, (1.0, (2 / (9 * ci)) ** 0.5, 1.0))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("channel_last", [False, True])
+def test_conv1d(channel_last, dtype):
+    """F.conv1d in both layouts and causal_conv1d_fn with SiLU."""
+    from amd_tuned_torch.causal_conv1d import causal_conv1d_fn
+
+    def lay(x):
+        return x.transpose(1, 2).contiguous().transpose(1, 2) if channel_last else x
+
+    def causal(x, w, b):
+        if x.is_cuda:
+            return causal_conv1d_fn(lay(x), w.squeeze(1), b, activation="silu")
+        return F.silu(F.conv1d(x, w, b, padding=3, groups=32)[..., :x.shape[2]])
+    shapes = ((2, 32, 67), (32, 1, 4), (32,))
+    _compare(lambda x, w, b: F.conv1d(lay(x), w, b, padding=3, groups=32), shapes, (2, 32, 70), dtype, (1.0, 0.5, 0.1))
+    _compare(causal, shapes, (2, 32, 67), dtype, (1.0, 0.5, 0.1))
+
+
 def _bar(got, ref, dtype):
     err = (got.detach().double().cpu() - ref.detach()).abs().max().item() / ref.abs().max().item()
     assert err <= (1e-5 if dtype == torch.float32 else 1e-2), err
