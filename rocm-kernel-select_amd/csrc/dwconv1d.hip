@@ -1583,7 +1583,7 @@ extern "C" int atk_causal_conv1d_bwd(const void* x, const void* dout, const void
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dout) | reinterpret_cast<uintptr_t>(dx)) & (es - 1))
     return fail(ATK_EINVAL, "causal_conv1d_bwd: misaligned element pointer");
   const int64_t rows = B * D;
-  if (rows >= (1ll << 31) || L >= (1ll << 31) / es - 64) return fail(ATK_UNSUPPORTED, "causal_conv1d_bwd: too large");
+  if (rows >= (1ll << 31) || L >= (1ll << 31) / es) return fail(ATK_UNSUPPORTED, "causal_conv1d_bwd: too large");
   const size_t need = (size_t)rows * (size_t)(K + 1) * sizeof(float);
   if (!workspace || ws_bytes < need) return fail(ATK_EINVAL, "causal_conv1d_bwd: workspace of %zu bytes needed", need);
   CrArgs a{};

@@ -10,6 +10,7 @@ import re
 import subprocess
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "amd_tuned_torch_hip.h")
@@ -150,6 +151,16 @@ def test_group_norm_backward_refuses_unaligned_rows_in_place(nat):
         assert lib.atk_group_norm_bwd(x, dy, None, dx, None, None, 2, 4, 7, 2, 1e-5, 0, 0, ws, ws_bytes,
                                       None) == nat.ATK_UNSUPPORTED
         assert "in place" in nat.last_error()
+
+
+def test_causal_backward_takes_rows_up_to_2gib(nat):
+    """The longest rows that the forward takes get past the size check (to the missing workspace);
+    rows of 2 GiB do not.  Host checks only: the pointers are never read."""
+    lib = nat.lib()
+    p = 1 << 20
+    for L, code in (((1 << 30) - 8, nat.ATK_EINVAL), (1 << 30, nat.ATK_UNSUPPORTED)):
+        assert lib.atk_causal_conv1d_bwd(p, p, p, None, p, p, None, 1, 1, L, 4, 4, 1, nat._DTYPE_CODE[torch.bfloat16],
+                                         0, 0, None, 0, None) == code, nat.last_error()
 
 
 def _fastdiv(n, d):
