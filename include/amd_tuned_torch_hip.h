@@ -518,7 +518,7 @@ int atk_conv_wgrad(const void* x, const void* dy, float* dw, int64_t N, int64_t 
 
 /* The same weight gradient, and the bias gradient db[co] = sum_{n,z,y,x} dy[n,co,z,y,x] when db
  * is not null, from one pass over x and dy.  Any Ci and Co, any W >= 8, rows of any alignment,
- * tensors under 2 GiB.  dw [Co, Ci, KD, 3, 3] and db [Co] are out_dtype: ATK_F32, or dtype
+ * H and W under 2^24, tensors under 2 GiB.  dw [Co, Ci, KD, 3, 3] and db [Co] are out_dtype: ATK_F32, or dtype
  * (the fp32 sums rounded once).  ATK_UNSUPPORTED (and 0 workspace bytes) outside that. */
 size_t atk_conv_param_grads_workspace_bytes(int64_t N, int64_t Ci, int64_t D, int64_t H, int64_t W, int64_t Co,
                                             int KD);

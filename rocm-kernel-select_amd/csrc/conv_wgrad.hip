@@ -746,7 +746,9 @@ bool wgrad_takes(int64_t N, int64_t Ci, int64_t Co, int64_t D, int64_t H, int64_
     if (v >= lim || pos >= lim) return false;
     pos *= v;
   }
-  return pos < lim && Ci < lim && Co < lim && pos * Ci < lim && pos * Co < lim && Ci * Co < lim / 27;
+  // (rows and columns within the 24 bits of chunk_off's product)
+  return H < (1 << 24) && W < (1 << 24) && pos < lim && Ci < lim && Co < lim && pos * Ci < lim && pos * Co < lim &&
+         Ci * Co < lim / 27;
 }
 
 // Shapes of conv_wgrad_rows_kernel, and the limits of atk_conv_wgrad.

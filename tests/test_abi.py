@@ -191,6 +191,17 @@ def test_conv_wgrad_workspace_query_declines_unserved_shapes(nat):
     assert L.atk_conv_wgrad_workspace_bytes(1, 256, 8, 64, 64, 256, 3) > 0
 
 
+def test_conv_param_grads_limits(nat):
+    """Planes whose row offsets leave the kernel's 24-bit product are declined, by the size query and
+    by the launch (host checks only)."""
+    lib = nat.lib()
+    for H, W, taken in ((1 << 24, 8, False), (2, 1 << 24, False), ((1 << 24) - 1, 8, True), (2, (1 << 24) - 8, True)):
+        assert (lib.atk_conv_param_grads_workspace_bytes(1, 1, 1, H, W, 1, 1) > 0) == taken
+        if not taken:
+            assert lib.atk_conv_param_grads(1 << 20, 1 << 20, 1 << 20, None, 1, 1, 1, H, W, 1, 1, 1, 0, None, 0,
+                                            None) == nat.ATK_UNSUPPORTED
+
+
 def test_argument_block_layouts_match_the_header(nat, tmp_path):
     """The ctypes mirrors of atk_dwconv1d_args / atk_group_norm_args / atk_conv_prepacked_args
     have the C compiler's size and field offsets (a C program compiled against the header
