@@ -38,6 +38,7 @@
 // fp16 29 us, of which the partials of 128 chunks are a third; 5x96x12x11x30 -> 192 62 us
 // against 298 us.  Before this kernel all of these took aten's backward.
 #include <algorithm>
+#include <atomic>
 
 #include "conv_common.h"
 
@@ -772,10 +773,16 @@ size_t workspace_bytes(int64_t N, int64_t Ci, int64_t Co, int64_t D, int64_t H, 
 // The kernels use more than the default 64 KB of dynamic LDS.
 template <typename T, int WCO, bool RAG>
 int launch_main(const WgArgs& a, dim3 grid, size_t lds, hipStream_t s) {
-  if (lds > 64 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_wgrad_kernel<T, WCO, RAG>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, WG_LDS_MAX);
-    if (e != hipSuccess) return fail(ATK_ELAUNCH, "conv_wgrad: cannot raise the LDS limit (%s)", hipGetErrorString(e));
+  if (lds > 64 * 1024) {  // raised once per kernel and device
+    static std::atomic<uint64_t> raised{0};
+    int dev = 0;
+    const uint64_t bit = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 ? 1ull << dev : 0;
+    if (!(raised.load(std::memory_order_relaxed) & bit)) {
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_wgrad_kernel<T, WCO, RAG>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, WG_LDS_MAX);
+      if (e != hipSuccess) return fail(ATK_ELAUNCH, "conv_wgrad: cannot raise the LDS limit (%s)", hipGetErrorString(e));
+      raised.fetch_or(bit, std::memory_order_relaxed);
+    }
   }
   hipLaunchKernelGGL((conv_wgrad_kernel<T, WCO, RAG>), grid, dim3(WG_NT), lds, s, a);
   return check_launch("conv_wgrad_kernel");
