@@ -544,6 +544,58 @@ def test_conv_param_grads_match_float64(case, dtype):
     assert torch.equal(_native.conv_wgrad(x.cuda(), dy.cuda(), KD), dw)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [(1, 32, 128, 1, 5, 16, 1), (2, 64, 256, 3, 9, 48, 3)])
+def test_conv_wgrad_entry_point(case, dtype):
+    """atk_conv_wgrad through the C ABI: the bits of atk_conv_param_grads without db in fp32, and its
+    refusal of a misaligned tensor and of shapes off its tiles."""
+    nat = _native()
+    N, Ci, Co, D, H, W, KD = case
+    g = torch.Generator().manual_seed(W)
+    x = torch.randn(N, Ci, D, H, W, generator=g).to(dtype).cuda()
+    dy = torch.randn(N, Co, D, H, W, generator=g).to(dtype).cuda()
+    lib = nat.lib()
+    ws = torch.empty(lib.atk_conv_wgrad_workspace_bytes(N, Ci, D, H, W, Co, KD), dtype=torch.uint8, device="cuda")
+    dw = torch.empty(Co, Ci, KD, 3, 3, device="cuda")
+
+    def call(px, ci=Ci):
+        return lib.atk_conv_wgrad(px, dy.data_ptr(), dw.data_ptr(), N, ci, D, H, W, Co, KD, nat._DTYPE_CODE[dtype],
+                                  ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert call(x.data_ptr()) == nat.ATK_OK
+    assert torch.equal(dw, nat.conv_wgrad(x, dy, KD))
+    assert call(x.data_ptr() + 2) == nat.ATK_UNSUPPORTED and call(x.data_ptr(), 16) == nat.ATK_UNSUPPORTED
+
+
+# Dilated planes: the patch's halo, the tile rectangle and the unaligned rows' partial chunks with
+# dilation 2 and 3, along either axis alone
+DILATED_CASES = [
+    (1, 16, 32, 9, 13, (1, 1), (2, 2), (2, 2)),
+    (2, 40, 96, 33, 45, (1, 1), (2, 2), (2, 2)),
+    (1, 24, 64, 20, 80, (1, 1), (1, 3), (1, 3)),
+    (1, 32, 40, 17, 31, (1, 1), (3, 2), (3, 2)),
+    (1, 64, 128, 24, 40, (1, 1), (2, 2), (2, 2)),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("case", DILATED_CASES, ids=lambda c: "x".join(map(str, c[:5])) + f"_s{c[5][0]}_d{c[7][0]}{c[7][1]}")
+def test_conv2d_dilated_every_tile(case, dtype):
+    """Every tile that takes the shape against the float64 oracle."""
+    nat = _native()
+    N, Ci, Co, H, W, s, p, d = case
+    x, w, b = _inputs((N, Ci, H, W), (Co, Ci, 3, 3), dtype, seed=H + W)
+    ref = torch.nn.functional.conv2d(x.double(), w.double(), b.double(), s, p, d)
+    ran = 0
+    for vi, name in enumerate(nat.variants(nat.OP_CONV)):
+        try:
+            y = nat.conv2d(x.cuda(), w.cuda(), b.cuda(), s, p, d, variant=vi)
+        except nat.Unsupported:
+            continue
+        ran += 1
+        assert O.max_rel_err(y.cpu(), ref) <= BAR[dtype], name
+    assert ran >= 2
+
+
 @pytest.mark.parametrize("W", [13, 16])
 def test_conv_param_grads_keep_infinities_local(W):
     """An infinity in x reaches only the gradients whose sums contain it: the tap that would
