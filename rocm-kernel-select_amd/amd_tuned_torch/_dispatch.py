@@ -406,10 +406,9 @@ def _dgrad_via_forward(grad_output, weight, pad_t, nd, fwd):
     return fwd(dy, wt, None, 1, pad_t, 1, 1)
 
 
-def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd, bias_grad):
-    """(dw, db) through the native kernel for stride-1, dilation-1, groups-1 'same' convs with
-    3x3 (2D) or 3x3x3 / 1x3x3 (3D) kernels in 16-bit types, db (the sum of dy, in the weight's
-    dtype) only with `bias_grad`; None otherwise (or when the kernel declines the shape)."""
+def _wgrad_operands(input, grad_output, weight, stride, padding, dilation, groups, nd):
+    """(x, dy, kernel depth) of the native weight gradient, 5-D: stride-1, dilation-1, groups-1 'same'
+    convs with 3x3 (2D) or 3x3x3 / 1x3x3 (3D) kernels in 16-bit types; None otherwise."""
     if (groups != 1 or isinstance(padding, str) or weight.dtype not in (torch.float16, torch.bfloat16)
             or not _native.available()):
         return None
@@ -431,6 +430,13 @@ def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups,
         kd, x5, g5 = 1, input.unsqueeze(2), grad_output.unsqueeze(2)
     if g5.dtype != x5.dtype or tuple(g5.shape[2:]) != tuple(x5.shape[2:]):
         return None
+    return x5, g5, kd
+
+
+def _wgrad_native(operands, weight, bias_grad):
+    """(dw, db) of _wgrad_operands through the native kernel, db (the sum of dy, in the weight's
+    dtype) only with `bias_grad`; None when the kernel declines the shape."""
+    x5, g5, kd = operands
     out_dtype = weight.dtype if weight.dtype == x5.dtype else torch.float32
     try:
         got = _native.conv_wgrad(_to_ncdhw(x5), _to_ncdhw(g5), kd, bias_grad=bias_grad, out_dtype=out_dtype)
@@ -440,11 +446,60 @@ def _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups,
     return dw.view(weight.shape).to(weight.dtype), None if db is None else db.to(weight.dtype)
 
 
+def _wgrad_contested(weights: int, positions: int) -> bool:
+    """Whether the native weight gradient and aten's are contested for a shape.  The kernel writes and
+    re-reads fp32 partials of every weight however few positions there are, so many channels on a
+    small plane can be faster in aten's GEMM: bf16 with db, native against aten, 2-D 2048 -> 2048 on
+    1x12x12 203 and 91 us (4x8x8: 245 and 378), 1280 -> 1280 on 2x45x45 336 and 213 (4x24x24: 182 and
+    246), 3-D 1280 -> 640 on 4x8x8 143 and 83 (4 samples of 4x24x24: 736 and 1407).  With fewer than
+    2^23 weights the native kernel was ahead, or within 1 %, at all of 140 sizes.  With up to 2^24
+    and few positions both are shorter than their host calls, of which aten's takes 50 us more (a
+    backward of 1280 -> 1280 on 8x8 159 us, by aten 211, though its kernels take 56 against 85)."""
+    return weights >= 1 << 24 or (weights >= 1 << 23 and positions >= 2048)
+
+
+def _weight_grads(grad_output, input, weight, bias_sizes, conf, bias_grad):
+    """(dw, db) of a conv by the native kernel or, where that is contested and lost, by aten; None
+    where neither a kernel nor a contest serves the shape."""
+    operands = _wgrad_operands(input, grad_output, weight, *conf)
+    if operands is None:
+        return None
+    if (not _wgrad_contested(weight.numel(), grad_output.numel() // weight.shape[0]) or not kernel_select.enabled()
+            or weight.dtype != input.dtype):
+        return _wgrad_native(operands, weight, bias_grad)
+    got = {}
+
+    def native():
+        got[_NATIVE_PREFIX + "wgrad"] = r = _wgrad_native(operands, weight, bias_grad)
+        return None if r is None else r[0]
+
+    def stock():
+        got["stock"] = r = _aten_conv_grads(grad_output, input, weight, bias_sizes, conf, [False, True, bias_grad])[1:]
+        return r[0]
+
+    key = (conf[4], input.dtype, tuple(input.shape), tuple(weight.shape), _channels_last(input),
+           _channels_last(grad_output), bool(bias_grad))
+    dw = kernel_select.pick_key("conv_wgrad", key, [(_NATIVE_PREFIX + "wgrad", native), ("stock", stock)])
+    for r in got.values():
+        if r is not None and r[0] is dw:
+            return r
+    return _wgrad_native(operands, weight, bias_grad)
+
+
+def _aten_conv_grads(grad_output, input, weight, bias_sizes, conf, needs):
+    stride, padding, dilation, groups, nd = conf
+    tup = _triple if nd == 3 else _pair
+    return torch.ops.aten.convolution_backward(
+        grad_output.contiguous(), input, weight, bias_sizes, list(tup(stride)), list(tup(padding)),
+        list(tup(dilation)), False, [0] * nd, groups, needs)
+
+
 def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
     """(dx, dw, db) of a patched conv for `needs` = [dx, dw, db] wanted:
     * dx of a stride-1, dilation-1, groups-1 conv through `fwd` (the accelerated forward) on dy
       with transposed, flipped weights;
-    * dw of a 'same' 3x3(x3) conv in a 16-bit type through the native wgrad kernel, db with it;
+    * dw of a 'same' 3x3(x3) conv in a 16-bit type through the native wgrad kernel, db with it (for
+      many weights where it wins the shape's contest against aten);
     * db alone as a reduction of dy once every other gradient is native;
     * whatever is left, and everything that must be differentiable itself (graph_wanted), through
       aten.convolution_backward, the op autograd uses unpatched."""
@@ -461,7 +516,7 @@ def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
             else:
                 gi = None
     if needs[1] and native:
-        got = _wgrad_native(input, grad_output, weight, stride, padding, dilation, groups, nd, needs[2])
+        got = _weight_grads(grad_output, input, weight, bias_sizes, conf, needs[2])
         if got is not None:
             gw, gb = got
             needs[1] = False
@@ -470,10 +525,7 @@ def _conv_grads(grad_output, input, weight, bias_sizes, conf, needs, fwd):
         gb = grad_output.sum(dim=[0] + list(range(2, 2 + nd)), dtype=torch.float32).to(weight.dtype)
         needs[2] = False
     if any(needs):
-        tup = _triple if nd == 3 else _pair
-        ai, aw, ab = torch.ops.aten.convolution_backward(
-            grad_output.contiguous(), input, weight, bias_sizes, list(tup(stride)),
-            list(tup(padding)), list(tup(dilation)), False, [0] * nd, groups, needs)
+        ai, aw, ab = _aten_conv_grads(grad_output, input, weight, bias_sizes, conf, needs)
         gi = ai if gi is None else gi
         gw = aw if gw is None else gw
         gb = ab if gb is None else gb

@@ -528,6 +528,59 @@ def test_conv_backward_without_the_library(monkeypatch, dtype):
         assert (a.as_subclass(torch.Tensor).double() - r).abs().max() <= bar * r.abs().max()
 
 
+@pytest.mark.parametrize("bias_grad", [True, False])
+@pytest.mark.parametrize("faster", ["native.wgrad", "stock"])
+def test_weight_gradient_contest_for_many_weights(monkeypatch, contest, faster, bias_grad):
+    """For many weights the faster of the native kernel and aten serves the weight and bias gradients,
+    decided once per shape; fewer weights go native without a contest."""
+    calls = []
+    g = torch.Generator().manual_seed(9)
+    x, dy = (torch.randn(2, c, 9, 10, generator=g).to(torch.bfloat16) for c in (4, 6))
+    w = torch.randn(6, 4, 3, 3, generator=g).to(torch.bfloat16)
+    conf = (1, 1, 1, 1, 2)
+
+    def aten(grad_output, input, weight, bias_sizes, conf, needs):
+        calls.append("stock")
+        assert needs == [False, True, bias_grad]
+        return real(grad_output, input, weight, bias_sizes, conf, needs)
+
+    def wgrad(x5, g5, kd, *, bias_grad, out_dtype):
+        calls.append("native.wgrad")
+        _, dw, db = real(dy, x, w, [6], conf, [False, True, True])
+        return (dw, db) if bias_grad else dw
+    real = _dispatch._aten_conv_grads
+    monkeypatch.setattr(_native, "available", lambda: True)
+    monkeypatch.setattr(_native, "conv_wgrad", wgrad)
+    monkeypatch.setattr(_dispatch, "_aten_conv_grads", aten)
+    ref = real(dy, x, w, [6], conf, [False, True, bias_grad])[1:]
+
+    def run():
+        calls.clear()
+        got = _dispatch._weight_grads(dy, x, w, [6], conf, bias_grad)
+        torch.testing.assert_close(got[0], ref[0])
+        assert (got[1] is None) == (not bias_grad)
+        if bias_grad:
+            torch.testing.assert_close(got[1], ref[1])
+
+    run()
+    assert calls == ["native.wgrad"], "few weights: no contest"
+    assert not _dispatch._wgrad_contested((1 << 23) - 1, 1 << 20) and not _dispatch._wgrad_contested(1 << 23, 2047)
+    assert _dispatch._wgrad_contested(1 << 23, 2048) and _dispatch._wgrad_contested(1 << 24, 64)
+    monkeypatch.setattr(_dispatch, "_wgrad_contested", lambda weights, positions: (weights, positions) == (216, 180))
+    order = []
+
+    def fake_time(fn):
+        if fn() is None:
+            return None
+        order.append(calls[-1])
+        return 1.0 if calls[-1] == faster else 2.0
+    monkeypatch.setattr(kernel_select, "_time", fake_time)
+    run()
+    assert sorted(order) == ["native.wgrad", "stock"]
+    run()
+    assert calls == [faster], "the cached winner alone"
+
+
 def test_conv_dgrad_weight_declined_by_the_library(monkeypatch):
     """Too many weights for the kernel: the torch form."""
     class Lib:
