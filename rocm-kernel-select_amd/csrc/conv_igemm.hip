@@ -1823,8 +1823,11 @@ int launch_ig_vr(const IgPlan& pl, hipStream_t s) {
   return launch_ig_kern<conv_igemm_kernel<T, WCO, WSP, FCO, FSP, CB, XC, VR, KHT, KWT, false, KS>>(pl, nt, s);
 }
 
-// Tiles with an instantiation for unaligned rows under a 3x3 plane: the ones that win at some size
-// there; the others keep the element-wise loader.
+// Tiles with an instantiation for unaligned rows under a 3x3 plane: the ones that are the fastest of
+// all at some size there; the others keep the element-wise loader.  bf16, 150 random 2-D and 3-D
+// sizes of odd width, 32 to 512 channels, times each was first: w22_f11_cb32_ns 36, w22_f22_cb32 32,
+// w22_f11_cb32_k2 30, w14_f22_cb32 20, w22_f22_cb32_k2 19, w22_f24_cb16 6, w21_f14_cb32 6 (up to 11 % ahead
+// of the next), w22_f24_cb16_k2 1 (4 %).  fp32, 15 sizes: w22_f12_cb16 9, w22_f22_cb16 6.
 constexpr bool rag_tile(int wco, int wsp, int fco, int fsp, int cb, int xc, int ks, int es) {
   if (es == 4) return wco == 2 && ks == 1 && fco * fsp >= 2 && wsp == 2;
   if (xc != 1) return false;

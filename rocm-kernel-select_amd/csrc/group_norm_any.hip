@@ -290,10 +290,10 @@ int launch_any(const GaArgs& a, int64_t ngroups, int silu, hipStream_t s) {
 //          [1, 96, 96, 96], G = 1 with one value of 1e3, now 1e-7).
 //   apply: every workgroup merges its sample's records itself (the first rows of x are loaded
 //          before that), then normalises its chunk.
-// [16, 128, 64, 64] bf16 with SiLU: 73.9 us (stock: layout copies, moments, scale, SiLU) -> 15.0 us:
-// 6.4 the statistics (2.6 TB/s; 6.9 with the shifts waited for before the first rows were
-// requested), 9.1 the second pass (3.7 TB/s; 11.2 when the 16 parameters of a
-// thread were loaded one by one after the merge).
+// [16, 128, 64, 64] bf16 with SiLU: 73.9 us (stock: layout copies, moments, scale, SiLU) -> 13.4 us by
+// graph replay: 5.8 the statistics (2.9 TB/s; 6.2 with the chunk-wide shift, whose positions past
+// the chunk were computed and masked), 8.8 the second pass (3.8 TB/s; 11.2 when the 16 parameters
+// of a thread were loaded one by one after the merge).
 // ---------------------------------------------------------------------------------------
 constexpr int GC_NT = 256;
 constexpr int GC_MAXG = 256;
