@@ -157,7 +157,10 @@ def _grad_safe(*tensors: Any) -> bool:
     argument that requires grad (the reference's eligibility rule, _dispatch.py:528-553)."""
     if not torch.is_grad_enabled() or (_HAS_INFERENCE_MODE and torch.is_inference_mode_enabled()):
         return True
-    return not any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
+    for t in tensors:  # (a generator costs as much again)
+        if isinstance(t, torch.Tensor) and t.requires_grad:
+            return False
+    return True
 
 
 def _is_plain_tensor(t: Any) -> bool:
@@ -446,16 +449,21 @@ def _wgrad_native(operands, weight, bias_grad):
     return dw.view(weight.shape).to(weight.dtype), None if db is None else db.to(weight.dtype)
 
 
+# With fewer weights than this the native weight gradient was ahead of aten's, or within 1 %, at all of
+# 140 sizes, and is taken without a contest.
+_WGRAD_CONTEST = 1 << 23
+
+
 def _wgrad_contested(weights: int, positions: int) -> bool:
-    """Whether the native weight gradient and aten's are contested for a shape.  The kernel writes and
-    re-reads fp32 partials of every weight however few positions there are, so many channels on a
-    small plane can be faster in aten's GEMM: bf16 with db, native against aten, 2-D 2048 -> 2048 on
-    1x12x12 203 and 91 us (4x8x8: 245 and 378), 1280 -> 1280 on 2x45x45 336 and 213 (4x24x24: 182 and
-    246), 3-D 1280 -> 640 on 4x8x8 143 and 83 (4 samples of 4x24x24: 736 and 1407).  With fewer than
-    2^23 weights the native kernel was ahead, or within 1 %, at all of 140 sizes.  With up to 2^24
-    and few positions both are shorter than their host calls, of which aten's takes 50 us more (a
-    backward of 1280 -> 1280 on 8x8 159 us, by aten 211, though its kernels take 56 against 85)."""
-    return weights >= 1 << 24 or (weights >= 1 << 23 and positions >= 2048)
+    """Whether the native weight gradient and aten's are contested for a shape of _WGRAD_CONTEST weights
+    or more.  The kernel writes and re-reads fp32 partials of every weight however few positions
+    there are, so many channels on a small plane can be faster in aten's GEMM: bf16 with db, native
+    against aten, 2-D 2048 -> 2048 on 1x12x12 203 and 91 us (4x8x8: 245 and 378), 1280 -> 1280 on 2x45x45
+    336 and 213 (4x24x24: 182 and 246), 3-D 1280 -> 640 on 4x8x8 143 and 83 (4 samples of 4x24x24:
+    736 and 1407).  With up to 2^24 weights and few positions both are shorter than their host calls,
+    of which aten's takes 50 us more (a backward of 1280 -> 1280 on 8x8 159 us, by aten 211, though its
+    kernels take 56 against 85)."""
+    return weights >= 2 * _WGRAD_CONTEST or positions >= 2048
 
 
 def _weight_grads(grad_output, input, weight, bias_sizes, conf, bias_grad):
@@ -464,8 +472,9 @@ def _weight_grads(grad_output, input, weight, bias_sizes, conf, bias_grad):
     operands = _wgrad_operands(input, grad_output, weight, *conf)
     if operands is None:
         return None
-    if (not _wgrad_contested(weight.numel(), grad_output.numel() // weight.shape[0]) or not kernel_select.enabled()
-            or weight.dtype != input.dtype):
+    weights = weight.numel()
+    if (weights < _WGRAD_CONTEST or not _wgrad_contested(weights, grad_output.numel() // weight.shape[0])
+            or not kernel_select.enabled() or weight.dtype != input.dtype):
         return _wgrad_native(operands, weight, bias_grad)
     got = {}
 

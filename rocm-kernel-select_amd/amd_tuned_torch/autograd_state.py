@@ -8,7 +8,7 @@ from __future__ import annotations
 import torch
 import torch.autograd.forward_ad as _forward_ad
 
-_transform = torch._C._functorch.peek_interpreter_stack
+_transforming = torch._C._are_functorch_transforms_active
 _wrapped = torch._C._functorch.is_functorch_wrapped_tensor
 _grad_enabled = torch.is_grad_enabled
 
@@ -20,7 +20,7 @@ def _dual(tensors) -> bool:
 def transformed(*tensors) -> bool:
     """True when one of `tensors` (None and other values pass) carries a forward-mode tangent or is
     a functorch wrapper (vmap, jvp, grad)."""
-    if _forward_ad._current_level < 0 and _transform() is None:
+    if _forward_ad._current_level < 0 and not _transforming():
         return False
     if any(isinstance(t, torch.Tensor) and _wrapped(t) for t in tensors):
         return True

@@ -62,7 +62,10 @@ def _grad_safe(*tensors: Any) -> bool:
         return True
     if not torch.is_grad_enabled():
         return True
-    return not any(isinstance(t, torch.Tensor) and t.requires_grad for t in tensors)
+    for t in tensors:  # (a generator costs as much again)
+        if isinstance(t, torch.Tensor) and t.requires_grad:
+            return False
+    return True
 
 
 def _is_plain_tensor(t: Any) -> bool:

@@ -564,8 +564,9 @@ def test_weight_gradient_contest_for_many_weights(monkeypatch, contest, faster, 
 
     run()
     assert calls == ["native.wgrad"], "few weights: no contest"
-    assert not _dispatch._wgrad_contested((1 << 23) - 1, 1 << 20) and not _dispatch._wgrad_contested(1 << 23, 2047)
+    assert not _dispatch._wgrad_contested(1 << 23, 2047)
     assert _dispatch._wgrad_contested(1 << 23, 2048) and _dispatch._wgrad_contested(1 << 24, 64)
+    monkeypatch.setattr(_dispatch, "_WGRAD_CONTEST", 216)
     monkeypatch.setattr(_dispatch, "_wgrad_contested", lambda weights, positions: (weights, positions) == (216, 180))
     order = []
 
