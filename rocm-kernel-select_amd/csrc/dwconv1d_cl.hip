@@ -795,6 +795,7 @@ extern "C" size_t atk_dwconv1d_cl_bwd_weight_workspace_bytes(int64_t B, int64_t 
   using namespace atk;
   if (B <= 0 || D <= 0 || L_out <= 0 || K < 1 || !dtype_ok(dtype)) return 0;
   const int vec = 16 / (int)dtype_size(dtype);
+  if (D % vec) return 0;
   const uint32_t run = clw_run(B, D, L_out, vec);
   const int64_t nrw = (L_out + run - 1) / run;
   return (size_t)B * (size_t)nrw * (size_t)(K + 1) * (size_t)D * sizeof(float);
@@ -959,6 +960,7 @@ int cl_bwd_fused(const char* what, const void* x, const void* dout, const void* 
 extern "C" size_t atk_causal_conv1d_cl_bwd_workspace_bytes(int64_t B, int64_t D, int64_t L, int K, int dtype) {
   if (B <= 0 || D <= 0 || L <= 0 || K < 1 || !atk::dtype_ok(dtype)) return 0;
   const int vec = 16 / (int)atk::dtype_size(dtype);
+  if (D % vec) return 0;  // declined by the launch; without a whole vector there is no grid to size
   return atk::clb_workspace_bytes(B, D, K, atk::clb_span(B, D, L, K, K - 1, L, vec));
 }
 
@@ -982,6 +984,7 @@ extern "C" size_t atk_dwconv1d_cl_bwd_workspace_bytes(int64_t B, int64_t D, int6
       !atk::dtype_ok(dtype))
     return 0;
   const int vec = 16 / (int)atk::dtype_size(dtype);
+  if (D % vec) return 0;  // declined by the launch; without a whole vector there is no grid to size
   return atk::clb_workspace_bytes(B, D, K, atk::clb_span(B, D, L, K, pad_left, L_out, vec));
 }
 

@@ -191,6 +191,19 @@ def test_conv_wgrad_workspace_query_declines_unserved_shapes(nat):
     assert L.atk_conv_wgrad_workspace_bytes(1, 256, 8, 64, 64, 256, 3) > 0
 
 
+def test_channels_last_backward_sizes_decline_partial_vectors(nat):
+    """Channel counts that are no whole number of 16-byte vectors (fewer than one among them, which
+    divided by zero) size to 0, and the launches decline them."""
+    lib = nat.lib()
+    for dt, vec in (("float32", 4), ("float16", 8), ("bfloat16", 8)):
+        code = nat._DTYPE_CODE[getattr(torch, dt)]
+        for D in (1, vec - 1, vec + 1, vec, 2 * vec):
+            sizes = (lib.atk_causal_conv1d_cl_bwd_workspace_bytes(4, D, 100, 4, code),
+                     lib.atk_dwconv1d_cl_bwd_workspace_bytes(4, D, 100, 4, 3, 103, code),
+                     lib.atk_dwconv1d_cl_bwd_weight_workspace_bytes(4, D, 103, 4, code))
+            assert all((n > 0) == (D % vec == 0) for n in sizes), (dt, D, sizes)
+
+
 def test_conv_param_grads_limits(nat):
     """Planes whose row offsets leave the kernel's 24-bit product are declined, by the size query and
     by the launch (host checks only)."""
