@@ -468,13 +468,16 @@ def _wgrad_contested(weights: int, positions: int) -> bool:
 
 def _weight_grads(grad_output, input, weight, bias_sizes, conf, bias_grad):
     """(dw, db) of a conv by the native kernel or, where that is contested and lost, by aten; None
-    where neither a kernel nor a contest serves the shape."""
+    where neither a kernel nor a contest serves the shape.  A stream under capture is given the
+    kernel: a contest synchronises, which ends a capture, and aten's library call may clear memory
+    with nodes that a replay does not repeat rightly."""
     operands = _wgrad_operands(input, grad_output, weight, *conf)
     if operands is None:
         return None
     weights = weight.numel()
     if (weights < _WGRAD_CONTEST or not _wgrad_contested(weights, grad_output.numel() // weight.shape[0])
-            or not kernel_select.enabled() or weight.dtype != input.dtype):
+            or not kernel_select.enabled() or weight.dtype != input.dtype
+            or torch.cuda.is_current_stream_capturing()):
         return _wgrad_native(operands, weight, bias_grad)
     got = {}
 

@@ -532,7 +532,7 @@ def test_conv_backward_without_the_library(monkeypatch, dtype):
 @pytest.mark.parametrize("faster", ["native.wgrad", "stock"])
 def test_weight_gradient_contest_for_many_weights(monkeypatch, contest, faster, bias_grad):
     """For many weights the faster of the native kernel and aten serves the weight and bias gradients,
-    decided once per shape; fewer weights go native without a contest."""
+    decided once per shape; fewer weights, and a stream under capture, go native without a contest."""
     calls = []
     g = torch.Generator().manual_seed(9)
     x, dy = (torch.randn(2, c, 9, 10, generator=g).to(torch.bfloat16) for c in (4, 6))
@@ -552,6 +552,7 @@ def test_weight_gradient_contest_for_many_weights(monkeypatch, contest, faster, 
     monkeypatch.setattr(_native, "available", lambda: True)
     monkeypatch.setattr(_native, "conv_wgrad", wgrad)
     monkeypatch.setattr(_dispatch, "_aten_conv_grads", aten)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     ref = real(dy, x, w, [6], conf, [False, True, bias_grad])[1:]
 
     def run():
@@ -576,6 +577,10 @@ def test_weight_gradient_contest_for_many_weights(monkeypatch, contest, faster, 
         order.append(calls[-1])
         return 1.0 if calls[-1] == faster else 2.0
     monkeypatch.setattr(kernel_select, "_time", fake_time)
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        run()
+        assert calls == ["native.wgrad"] and not order, "no contest under capture"
     run()
     assert sorted(order) == ["native.wgrad", "stock"]
     run()
